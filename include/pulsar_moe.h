@@ -102,8 +102,9 @@ int pulsar_quantize_q8_K(void *out, const void *x, uint32_t in_dim, uint32_t n_r
 /* out[t][r] = sum_b dot(w row r block b, xq[t] block b), fp32 [n_tok][out_dim].
  * quant: the reference's dense list (pulsar_kernels.cu:5090-5142) - Q2_K,
  * IQ2_XXS, Q4_K, Q5_K, Q6_K, Q3_K, IQ4_XS, IQ4_NL, NVFP4 (the expert-only
- * formats return 0, as there); in_dim % 256 == 0. 5 or more tokens on Q4_K,
- * Q5_K, Q6_K or NVFP4 run the int8 matrix-core GEMM.
+ * formats return 0, as there); in_dim % 256 == 0. Chunks of 5 or more tokens
+ * run on the int8 matrix cores (IQ4_NL and the smallest chunks of the formats
+ * without a 16-row kernel excepted).
  * Replaces pulsar_matmul_kq (pulsar_kernels.cu:4895). */
 int pulsar_matmul_kq(void *out, const void *w, const void *xq, uint32_t in_dim,
                      uint32_t out_dim, uint32_t n_tok, uint64_t row_bytes,

@@ -14,8 +14,11 @@
 
 namespace pk {
 
-// mmq.hip: MFMA kernel for token chunks; returns -1 when it has no kernel
-// for the format (the caller then uses the lane kernels)
+// tile.hip, mmq.hip: matrix-core kernels for token chunks; -1 when one has no
+// kernel for the format or the shape (the caller then uses the next, and the
+// lane kernels last)
+int launch_tile_gemm(uint32_t quant, float *out, const uint8_t *w, const pulsar_block_q8_K *xq, uint32_t in_dim,
+                     uint32_t out_dim, uint32_t n_tok, uint64_t row_bytes);
 int launch_gemm(uint32_t quant, float *out, const uint8_t *w, const pulsar_block_q8_K *xq, uint32_t in_dim,
                 uint32_t out_dim, uint32_t n_tok, uint64_t row_bytes);
 
@@ -204,7 +207,8 @@ extern "C" int pulsar_matmul_kq(void *out, const void *w, const void *xq, uint32
     const uint8_t *wb = (const uint8_t *)w;
     const pulsar_block_q8_K *x = (const pulsar_block_q8_K *)xq;
     if (n_tok >= PK_MMQ_MIN_TOK) {
-        const int r = pk::launch_gemm(quant, o, wb, x, in_dim, out_dim, n_tok, row_bytes);
+        int r = pk::launch_tile_gemm(quant, o, wb, x, in_dim, out_dim, n_tok, row_bytes);
+        if (r < 0) r = pk::launch_gemm(quant, o, wb, x, in_dim, out_dim, n_tok, row_bytes);
         if (r >= 0) return r;
     }
     // the dense formats of pulsar_kernels.cu:5090-5142

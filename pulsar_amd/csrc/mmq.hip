@@ -1,9 +1,9 @@
 // mmq.hip - int8 matrix-core (v_mfma_i32_16x16x32_i8) kernels:
-//   mmq_gemm_kernel: the dense Q4_K / Q6_K matvec for token chunks and
-//     prefill (5 or more tokens; 16- or 32-token tiles). A block computes
-//     16 RT weight rows x 16 NT tokens; its waves split each K chunk's
-//     super-blocks and the partials are added in wave order through LDS
-//     (deterministic);
+//   mmq_gemm_kernel: the dense matvec for token chunks that tile.hip leaves
+//     (Q4_K, Q5_K, Q6_K: the smaller ones; NVFP4: all of 5 or more tokens). A
+//     block computes 16 RT weight rows x 16 NT tokens; its waves split each K
+//     chunk's super-blocks and the partials are added in wave order through
+//     LDS (deterministic);
 //   moe_grouped_mmq_kq_kernel: the grouped MoE stages (16 rows x up to 16
 //     (token, slot) pairs of one expert per MFMA tile) for Q2_K, IQ2_XXS,
 //     MXFP4, Q4_K, Q5_K and Q6_K experts.
@@ -528,9 +528,11 @@ static int launch_gemm_q(float *out, const uint8_t *w, const pulsar_block_q8_K *
     // 4096 11.1 -> 9.9 us, 14336 x 4096 19.2 -> 16.6 us; 5-31 tokens and
     // 14336-wide rows alike); Q6_K and NVFP4 spill at that cap (Q6_K 8192 x
     // 4096 12.8 -> 21.5 us)
-    if (n_tok >= PK_GEMM_NT2)
-        PK_GEMM(2, 2, 2, PK_GEMM_D_NT2);
-    else if (out_dim < 8192u)
+    // (Q4_K and Q5_K chunks of 17 or more tokens are tile.hip's)
+    constexpr bool kNt2 = Q != PULSAR_QUANT_Q4_K && Q != PULSAR_QUANT_Q5_K;
+    if (kNt2 && n_tok >= PK_GEMM_NT2) {
+        if constexpr (kNt2) PK_GEMM(2, 2, 2, PK_GEMM_D_NT2);
+    } else if (out_dim < 8192u)
         PK_GEMM(1, 8, 1, PK_GEMM_D_R16);
     else if (Q == PULSAR_QUANT_Q4_K)
         PK_GEMM(2, 8, 1, 1);
