@@ -600,25 +600,85 @@ namespace pk {
 template <typename G>
 int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, const float *weights,
                           const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
-                          uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes);
+                          uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
+                          uint32_t max_pairs);
 extern template int launch_grouped_mmq_kq<CsrGroups>(bool, uint32_t, float *, const CsrGroups &, const float *,
                                                      const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t,
-                                                     uint32_t, uint64_t, uint32_t, uint32_t);
+                                                     uint32_t, uint64_t, uint32_t, uint32_t, uint32_t);
 extern template int launch_grouped_mmq_kq<ExpertGroups>(bool, uint32_t, float *, const ExpertGroups &,
                                                         const float *, const pulsar_block_q8_K *, uint32_t, uint32_t,
-                                                        uint32_t, uint32_t, uint64_t, uint32_t, uint32_t);
+                                                        uint32_t, uint32_t, uint64_t, uint32_t, uint32_t, uint32_t);
+// tile_moe.hip: the grouped stages on the wide tile, for the groups of at
+// least min_pairs pairs
+uint32_t tile_min_quarter_pairs(bool pair, uint32_t quant);
+template <typename G>
+int launch_tile_grouped(bool pair, uint32_t quant, float *out, const G &src, const float *weights,
+                        const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
+                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
+                        uint32_t min_pairs);
+extern template int launch_tile_grouped<CsrGroups>(bool, uint32_t, float *, const CsrGroups &, const float *,
+                                                   const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t, uint32_t,
+                                                   uint64_t, uint32_t, uint32_t, uint32_t);
+extern template int launch_tile_grouped<ExpertGroups>(bool, uint32_t, float *, const ExpertGroups &, const float *,
+                                                      const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t, uint32_t,
+                                                      uint64_t, uint32_t, uint32_t, uint32_t);
+
+// The routed pairs of an ExpertGroups stage and the experts they spread over at
+// most (a caller's CSR: unknown on the host).
+struct GroupSizes {
+    uint32_t routed = 0, experts = 1;
+};
+
+// A grouped stage on the matrix cores; -1 where only the lane kernels have the
+// format. The routed experts' mean decides between the two kernels; a shared
+// slot's group, which holds every token, goes to the tile by its own size (top-8
+// of 256 experts and a shared one, 128 tokens: its 8 pair tiles one after the
+// other made the gate / up stage 331 us, now 142). The sizes in a caller's CSR are not known here: those stay
+// with the kernel made for short groups where there is one.
+template <typename G>
+static int grouped_mfma(bool pair, uint32_t quant, float *out, const G &grp, const float *weights,
+                        const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
+                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
+                        const GroupSizes &sizes) {
+    // rows wider than the lane kernels take are refused for every format
+    const uint32_t bound = k_dim <= 16384u ? tile_min_quarter_pairs(pair, quant) : 0u;
+    auto tile = [&](const G &src, uint32_t groups) {
+        return launch_tile_grouped(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, groups, row_bytes,
+                                   act_op, lst_bytes, 0u);
+    };
+    auto mmq = [&](const G &src) {
+        return launch_grouped_mmq_kq(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, n_group, row_bytes,
+                                     act_op, lst_bytes, UINT32_MAX);
+    };
+    if (bound == 0u) return mmq(grp);
+    if constexpr (std::is_same<G, ExpertGroups>::value) {
+        if (4u * sizes.routed >= bound * sizes.experts) return tile(grp, n_group);
+        if (grp.n_shared != 0u && grp.n_tok >= (pair ? 33u : 100u)) {
+            G part = grp;
+            part.which = ExpertGroups::kRouted;
+            const int r = mmq(part);
+            if (r <= 0) return r < 0 ? mmq(grp) : r;
+            part.which = ExpertGroups::kShared;
+            return tile(part, grp.n_shared);
+        }
+        return mmq(grp);
+    } else {
+        const int r = mmq(grp);
+        return r < 0 && (quant == PULSAR_QUANT_Q3_K || quant == PULSAR_QUANT_IQ4_XS) ? tile(grp, n_group) : r;
+    }
+}
 
 // The grouped gate / up stage for either group source: the matrix-core
-// kernel where the format has one, else the lane kernels.
+// kernels where the format has one, else the lane kernels.
 template <typename G>
 static int pair_grouped(void *mid, const G &grp, const void *weights, const void *xq, uint32_t in_dim,
                         uint32_t mid_dim, uint32_t n_used, uint32_t n_group, uint64_t row_bytes, uint32_t quant,
-                        uint32_t act_op, uint32_t lst_bytes) {
+                        uint32_t act_op, uint32_t lst_bytes, const GroupSizes &sizes = {}) {
 #ifndef PK_GRP_LANE_ONLY
     {
-        const int r = launch_grouped_mmq_kq(true, quant, (float *)mid, grp, (const float *)weights,
-                                            (const pulsar_block_q8_K *)xq, in_dim, mid_dim, n_used, n_group,
-                                            row_bytes, act_op, lst_bytes);
+        const int r = grouped_mfma(true, quant, (float *)mid, grp, (const float *)weights,
+                                   (const pulsar_block_q8_K *)xq, in_dim, mid_dim, n_used, n_group, row_bytes, act_op,
+                                   lst_bytes, sizes);
         if (r >= 0) return r;
     }
 #endif
@@ -630,12 +690,12 @@ static int pair_grouped(void *mid, const G &grp, const void *weights, const void
 
 template <typename G>
 static int down_grouped(void *partial, const G &grp, const void *midq, uint32_t mid_dim, uint32_t out_dim,
-                        uint32_t n_used, uint32_t n_group, uint64_t row_bytes, uint32_t quant, uint32_t lst_bytes) {
+                        uint32_t n_used, uint32_t n_group, uint64_t row_bytes, uint32_t quant, uint32_t lst_bytes,
+                        const GroupSizes &sizes = {}) {
 #ifndef PK_GRP_LANE_ONLY
     {
-        const int r = launch_grouped_mmq_kq(false, quant, (float *)partial, grp, nullptr,
-                                            (const pulsar_block_q8_K *)midq, mid_dim, out_dim, n_used, n_group,
-                                            row_bytes, 0, lst_bytes);
+        const int r = grouped_mfma(false, quant, (float *)partial, grp, nullptr, (const pulsar_block_q8_K *)midq,
+                                   mid_dim, out_dim, n_used, n_group, row_bytes, 0u, lst_bytes, sizes);
         if (r >= 0) return r;
     }
 #endif
@@ -708,9 +768,11 @@ static bool experts_args_ok(const void *selected, const void *active, const puls
 
 // The grid's group count: every expert the chunk can touch, the shared
 // slots and the NULL group (groups past the touched count are empty).
+static uint32_t touched_groups(uint32_t n_expert, uint32_t n_tok, uint32_t k_used) {
+    return n_tok * k_used < n_expert ? n_tok * k_used : n_expert;
+}
 static uint32_t expert_grid_groups(uint32_t n_expert, uint32_t n_shared, uint32_t n_tok, uint32_t k_used) {
-    const uint32_t touch = n_tok * k_used < n_expert ? n_tok * k_used : n_expert;
-    return touch + n_shared + 1u;
+    return touched_groups(n_expert, n_tok, k_used) + n_shared + 1u;
 }
 
 extern "C" int pulsar_moe_pair_swiglu_experts(void *mid, const void *selected, const void *active,
@@ -729,7 +791,7 @@ extern "C" int pulsar_moe_pair_swiglu_experts(void *mid, const void *selected, c
     const ExpertGroups grp = expert_groups(selected, active, bank, n_expert, shared, n_shared, n_tok, k_used);
     return pair_grouped(mid, grp, slot_weights, xq, in_dim, mid_dim, k_used + n_shared,
                         expert_grid_groups(n_expert, n_shared, n_tok, k_used), row_bytes, quant, act_op,
-                        4u * n_tok * k_used);
+                        4u * n_tok * k_used, GroupSizes{n_tok * k_used, touched_groups(n_expert, n_tok, k_used)});
 }
 
 extern "C" int pulsar_moe_down_experts(void *partial, const void *selected, const void *active, const void *midq,
@@ -745,7 +807,7 @@ extern "C" int pulsar_moe_down_experts(void *partial, const void *selected, cons
     const ExpertGroups grp = expert_groups(selected, active, bank, n_expert, shared, n_shared, n_tok, k_used);
     return down_grouped(partial, grp, midq, mid_dim, out_dim, k_used + n_shared,
                         expert_grid_groups(n_expert, n_shared, n_tok, k_used), row_bytes, quant,
-                        4u * n_tok * k_used);
+                        4u * n_tok * k_used, GroupSizes{n_tok * k_used, touched_groups(n_expert, n_tok, k_used)});
 }
 
 extern "C" int pulsar_moe_slot_sum(void *out, const void *partial, uint32_t out_dim, uint32_t n_used,

@@ -345,6 +345,7 @@ struct CsrGroups {
         e = starts[G.g + 1u];
     }
     PK_DEV uint32_t pair(uint32_t i, const uint32_t *) const { return pairs[i]; }
+    PK_DEV void range_block(const Group &G, uint32_t *lst, uint32_t &b, uint32_t &e) const { range(G, lst, b, e); }
 };
 
 // One group per expert a chunk touches, in a resident bank, found from the
@@ -367,6 +368,9 @@ struct ExpertGroups {
     pulsar_expert_bank bank;
     SharedSlots shared;
     uint32_t n_expert, k_used, n_shared, n_tok;
+    // which groups a launch is for: all, all but the shared slots' (empty
+    // here), or the shared slots' alone (group g is shared slot g)
+    enum Part : uint32_t { kAll, kRouted, kShared } which;
     struct Group {
         pulsar_expert_ptrs p;
         uint32_t kind, e;  // kind 0: routed expert e, 1: shared slot e, 2: NULL, 3: empty
@@ -386,12 +390,16 @@ struct ExpertGroups {
         G.pf[1] = sel[lane + 64u < total ? lane + 64u : total - 1u];
         G.p = pulsar_expert_ptrs{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
         G.e = 0u;
-        if (g < n_act) {
+        if (which == kShared) {
+            G.kind = 1u;
+            G.e = g;
+            G.p = shared.p[g];
+        } else if (g < n_act) {
             G.kind = 0u;
             G.e = e_g;
             G.p = bank_ptrs(bank, n_expert, (int32_t)e_g);
         } else if (g < n_act + n_shared) {
-            G.kind = 1u;
+            G.kind = which == kRouted ? 3u : 1u;
             G.e = g - n_act;
             G.p = shared.p[G.e];
         } else {
@@ -435,6 +443,58 @@ struct ExpertGroups {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     PK_DEV uint32_t pair(uint32_t i, const uint32_t *lst) const { return lst[i]; }
+    // range() by a whole block of 4 waves: each scans a quarter of the ids, all
+    // its loads in flight at once, and the quarters' counts place their hits.
+    // One round trip and two block barriers, where a wave that scans alone
+    // takes one dependent step per 64 ids (2048 ids: ~20 us of a stage). Every
+    // thread of the block calls it; the list is readable on return.
+    PK_DEV void range_block(const Group &G, uint32_t *lst, uint32_t &b, uint32_t &e) const {
+        constexpr uint32_t kStrips = 8u;  // 2048 ids / (4 waves x 64 lanes)
+        __shared__ uint32_t count[4];
+        const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        b = e = 0u;
+        if (G.kind == 3u) return;  // block-uniform
+        if (G.kind == 1u) {
+            for (uint32_t t = threadIdx.x; t < n_tok; t += 256u) lst[t] = (t << 4) | (k_used + G.e);
+            e = n_tok;
+        } else {
+            const bool nul = G.kind == 2u;
+            const uint32_t total = n_tok * k_used, strips = (total + 255u) / 256u, q0 = wave * strips * 64u + lane;
+            int32_t id[kStrips];
+#pragma unroll
+            for (uint32_t k = 0; k < kStrips; k++)
+                if (k < strips) id[k] = sel[q0 + 64u * k < total ? q0 + 64u * k : total - 1u];
+            uint64_t bal[kStrips];
+            uint32_t mine = 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < kStrips; k++) {
+                bal[k] = 0u;
+                if (k < strips) {
+                    const bool hit = q0 + 64u * k < total &&
+                                     (nul ? (id[k] < 0 || (uint32_t)id[k] >= n_expert) : id[k] == (int32_t)G.e);
+                    bal[k] = __ballot(hit);
+                    mine += (uint32_t)__builtin_popcountll(bal[k]);
+                }
+            }
+            if (lane == 0u) count[wave] = mine;
+            __syncthreads();
+            uint32_t at = 0u;
+#pragma unroll
+            for (uint32_t w = 0; w < 4u; w++) {
+                at += w < wave ? count[w] : 0u;
+                e += count[w];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kStrips; k++) {
+                if (bal[k] >> lane & 1u) {
+                    const uint32_t q = q0 + 64u * k, t = q / k_used;
+                    lst[at + (uint32_t)__builtin_popcountll(bal[k] & ((1ull << lane) - 1ull))] = (t << 4) | (q - t * k_used);
+                }
+                at += (uint32_t)__builtin_popcountll(bal[k]);
+            }
+        }
+        __syncthreads();
+    }
 };
 
 }  // namespace pk

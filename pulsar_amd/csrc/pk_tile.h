@@ -429,11 +429,11 @@ struct Tile {
 
     float acc[NS][2][4];  // [slice][row tile][token 4q + r]
 
-    // w[rt]: the lane's two weight rows; xb + off_of(t): the q8_K row of token
+    // w0, w1: the lane's two weight rows; xb + off_of(t): the q8_K row of token
     // t < np (0 < np <= kTok); buf0, buf1: kBuf bytes each, two distinct LDS
-    // arrays. On return the lanes of wave (wr, wk) hold the sums of their
-    // share of the elements (mine()).
-    template <typename OffOf>
+    // arrays. NC: the token slices computed (16 NC >= np). On return the lanes
+    // of wave (wr, wk) hold the sums of their share of the elements (mine()).
+    template <uint32_t NC = NS, typename OffOf>
     PK_DEV void run(uint8_t *buf0, uint8_t *buf1, const uint2 *lut, const uint8_t *w0, const uint8_t *w1, uint32_t nb,
                     uint32_t np, const uint8_t *xb, OffOf off_of) {
         const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -442,7 +442,7 @@ struct Tile {
         // byte `at` of record rec of iteration it (tokens past np: the last one again)
         auto src = [&](uint32_t it, uint32_t rec, uint32_t at) {
             const uint32_t t = rec % kTok;
-            const uint32_t o = off_of(t < np ? t : np - 1u) + at;
+            const auto o = off_of(t < np ? t : np - 1u) + at;
             if constexpr (WK == 1u)
                 return (const PK_GLOBAL uint32_t *)(xb + clamp_sb(it) * 292u + o);
             else
@@ -526,8 +526,8 @@ struct Tile {
             v4i_t pl[2], ph[2];
             read_a(0u);
 #pragma unroll
-            for (uint32_t n = 0; n < NS; n++) {
-                if (n + 1u < NS) read_a(n + 1u);
+            for (uint32_t n = 0; n < NC; n++) {
+                if (n + 1u < NC) read_a(n + 1u);
                 v4i_t dl[2] = {}, dh[2] = {};
 #pragma unroll
                 for (uint32_t s = 0; s < 4; s++)
@@ -542,17 +542,8 @@ struct Tile {
                     pl[rt] = dl[rt];
                     ph[rt] = dh[rt];
                 }
-#ifdef PK_SGB
-                // one MFMA, then a few vector instructions of the previous slice
-#pragma unroll
-                for (uint32_t k = 0; k < (F::kHi ? 16u : 8u); k++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x102, PK_SGB, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#endif
             }
-            finish(NS - 1u, pl, ph);
+            finish(NC - 1u, pl, ph);
             arrived();
         };
         arrived();
@@ -569,13 +560,13 @@ struct Tile {
                 return (float *)(wv < 2u ? buf0 : buf1) + (((wv & 1u) * NS + n) * 8u + rt * 4u + r) * 64u + lane;
             };
 #pragma unroll
-            for (uint32_t n = 0; n < NS; n++)
+            for (uint32_t n = 0; n < NC; n++)
 #pragma unroll
                 for (uint32_t e = 0; e < 8; e++) *part(wave, n, e >> 2, e & 3u) = acc[n][e >> 2][e & 3u];
             __syncthreads();
             const uint32_t wr = wave % WR;
 #pragma unroll
-            for (uint32_t n = 0; n < NS; n++)
+            for (uint32_t n = 0; n < NC; n++)
 #pragma unroll
                 for (uint32_t e = 0; e < 8; e++)
                     if (mine(n, e & 3u, wk)) {
