@@ -266,9 +266,11 @@ int pulsar_moe_route(void *selected, void *weights, void *ptrs, void *slot_weigh
  * instead of a CSR (no reference counterpart: the reference groups on the
  * host, crates/engine/src/lib.rs:8357-8392). Each routed (token, slot)
  * pair runs in the group of its expert, shared slot i (s = k_used + i,
- * weight 1) of every token in a group of its own, exactly as
+ * weight 1) of every token in a group of its own, as
  * pulsar_moe_pair_swiglu_grouped / pulsar_moe_down_grouped would for the
- * same pairs, so the rows they write are bit-identical to those calls'.
+ * same pairs: the same exact integer sums, and the same rows bit for bit
+ * wherever both choose the same kernel by the groups' mean size (else their
+ * fp32 steps round differently in the last bits).
  * Slots whose id is outside [0, n_expert) get rows of 0 in mid (partial),
  * so every row of mid [n_tok][k_used + n_shared][mid_dim] (partial
  * [..][out_dim]) is written and partial needs no zeroing. slot_weights

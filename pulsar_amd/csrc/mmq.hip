@@ -759,7 +759,7 @@ template <uint32_t Q, bool PAIR, typename G>
 __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_eu(2))) void moe_grouped_mmq_kq_kernel(
         float *__restrict__ out, const G src, const float *__restrict__ weights,
         const pulsar_block_q8_K *__restrict__ act, uint32_t k_blocks, uint32_t lim, uint32_t n_rows,
-        uint32_t n_used, uint64_t row_bytes, uint32_t act_op, uint32_t pmax, uint32_t lst_off, uint32_t max_pairs) {
+        uint32_t n_used, uint64_t row_bytes, uint32_t act_op, uint32_t pmax, uint32_t lst_off, uint32_t bound) {
     using F = GmmqFmt<Q>;
     constexpr uint32_t NM = PAIR ? 2 : 1;
     constexpr bool kIq2 = Q == PULSAR_QUANT_IQ2_XXS;
@@ -786,6 +786,9 @@ __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_e
     }
     const uint32_t group = blockIdx.y;
     const typename G::Group grp = src.group(group);
+    // a caller's CSR whose groups are long on average is the wide tile's
+    if constexpr (std::is_same<G, CsrGroups>::value)
+        if (4ull * (src.starts[gridDim.y] - src.starts[0]) >= (uint64_t)bound * gridDim.y) return;
     const pulsar_expert_ptrs &p = grp.p;
     const uint8_t *w0 = PAIR ? (const uint8_t *)p.gate : (const uint8_t *)p.down;
     const uint8_t *w1 = PAIR ? (const uint8_t *)p.up : nullptr;
@@ -795,8 +798,6 @@ __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_e
     uint32_t s0, s1;
     src.range(grp, lst, s0, s1);
     if (s0 >= s1) return;
-    // a caller's CSR: the groups from max_pairs pairs on are the wide tile's
-    if (std::is_same<G, CsrGroups>::value && s1 - s0 >= max_pairs) return;
     if (nul) {  // unrouted slots: their rows of this block are 0
         const uint32_t nr = kGqBlockRows<Q, PAIR>, r0 = blockIdx.x * nr;
         for (uint32_t it = threadIdx.x; it < (s1 - s0) * nr; it += blockDim.x) {
@@ -1354,13 +1355,13 @@ __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_e
 // on the matrix cores; -1 for the other formats (the caller then uses the
 // lane kernels of moe.hip). `src` is the group source (CsrGroups or
 // ExpertGroups), n_group the grid's group count; lst_bytes the LDS the
-// source's pair list needs (0 for the caller's CSR). max_pairs: a CSR's groups
-// of that many pairs or more are left out.
+// source's pair list needs (0 for the caller's CSR). bound: a CSR whose
+// groups have bound / 4 pairs or more on average is left to the wide tile.
 template <typename G>
 int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, const float *weights,
                           const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
                           uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
-                          uint32_t max_pairs) {
+                          uint32_t bound) {
     if (quant != PULSAR_QUANT_Q2_K && quant != PULSAR_QUANT_IQ2_XXS && quant != PULSAR_QUANT_MXFP4 &&
         quant != PULSAR_QUANT_Q4_K && quant != PULSAR_QUANT_Q5_K && quant != PULSAR_QUANT_Q6_K)
         return -1;
@@ -1387,7 +1388,7 @@ int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, c
     hipLaunchKernelGGL((moe_grouped_mmq_kq_kernel<Q, P, G>),                                                     \
                        dim3((n_rows + kGqBlockRows<Q, P> - 1u) / kGqBlockRows<Q, P>, n_group),                     \
                        dim3(64u * kGqWaves<Q>), lds, pk::stream(), out, src, weights, act, k_blocks, lim, n_rows, \
-                       n_used, row_bytes, act_op, pmax, lst_off, max_pairs)
+                       n_used, row_bytes, act_op, pmax, lst_off, bound)
     if (quant == PULSAR_QUANT_Q2_K && pair)
         PK_GQ(PULSAR_QUANT_Q2_K, true);
     else if (quant == PULSAR_QUANT_Q2_K)

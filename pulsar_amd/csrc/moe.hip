@@ -608,20 +608,14 @@ extern template int launch_grouped_mmq_kq<CsrGroups>(bool, uint32_t, float *, co
 extern template int launch_grouped_mmq_kq<ExpertGroups>(bool, uint32_t, float *, const ExpertGroups &,
                                                         const float *, const pulsar_block_q8_K *, uint32_t, uint32_t,
                                                         uint32_t, uint32_t, uint64_t, uint32_t, uint32_t, uint32_t);
-// tile_moe.hip: the grouped stages on the wide tile, for the groups of at
-// least min_pairs pairs
+// tile_moe.hip: the grouped stages on the wide tile
 uint32_t tile_min_quarter_pairs(bool pair, uint32_t quant);
-template <typename G>
-int launch_tile_grouped(bool pair, uint32_t quant, float *out, const G &src, const float *weights,
+int launch_tile_experts(bool pair, uint32_t quant, float *out, const ExpertGroups &src, const float *weights,
                         const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
-                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
-                        uint32_t min_pairs);
-extern template int launch_tile_grouped<CsrGroups>(bool, uint32_t, float *, const CsrGroups &, const float *,
-                                                   const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t, uint32_t,
-                                                   uint64_t, uint32_t, uint32_t, uint32_t);
-extern template int launch_tile_grouped<ExpertGroups>(bool, uint32_t, float *, const ExpertGroups &, const float *,
-                                                      const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t, uint32_t,
-                                                      uint64_t, uint32_t, uint32_t, uint32_t);
+                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes);
+int launch_tile_csr(bool pair, uint32_t quant, float *out, const CsrGroups &src, const float *weights,
+                    const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used, uint32_t n_group,
+                    uint64_t row_bytes, uint32_t act_op, uint32_t bound);
 
 // The routed pairs of an ExpertGroups stage and the experts they spread over at
 // most (a caller's CSR: unknown on the host).
@@ -633,8 +627,9 @@ struct GroupSizes {
 // format. The routed experts' mean decides between the two kernels; a shared
 // slot's group, which holds every token, goes to the tile by its own size (top-8
 // of 256 experts and a shared one, 128 tokens: its 8 pair tiles one after the
-// other made the gate / up stage 331 us, now 142). The sizes in a caller's CSR are not known here: those stay
-// with the kernel made for short groups where there is one.
+// other made the gate / up stage 331 us, now 138). The sizes in a caller's
+// CSR are known on the device alone: both kernels are launched, and each works
+// or ends at once by the groups' mean.
 template <typename G>
 static int grouped_mfma(bool pair, uint32_t quant, float *out, const G &grp, const float *weights,
                         const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
@@ -642,29 +637,35 @@ static int grouped_mfma(bool pair, uint32_t quant, float *out, const G &grp, con
                         const GroupSizes &sizes) {
     // rows wider than the lane kernels take are refused for every format
     const uint32_t bound = k_dim <= 16384u ? tile_min_quarter_pairs(pair, quant) : 0u;
-    auto tile = [&](const G &src, uint32_t groups) {
-        return launch_tile_grouped(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, groups, row_bytes,
-                                   act_op, lst_bytes, 0u);
-    };
-    auto mmq = [&](const G &src) {
+    auto mmq = [&](const G &src, uint32_t b) {
         return launch_grouped_mmq_kq(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, n_group, row_bytes,
-                                     act_op, lst_bytes, UINT32_MAX);
+                                     act_op, lst_bytes, b);
     };
-    if (bound == 0u) return mmq(grp);
+    if (bound == 0u) return mmq(grp, UINT32_MAX);
     if constexpr (std::is_same<G, ExpertGroups>::value) {
+        auto tile = [&](const ExpertGroups &src, uint32_t groups) {
+            return launch_tile_experts(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, groups, row_bytes,
+                                       act_op, lst_bytes);
+        };
         if (4u * sizes.routed >= bound * sizes.experts) return tile(grp, n_group);
         if (grp.n_shared != 0u && grp.n_tok >= (pair ? 33u : 100u)) {
             G part = grp;
             part.which = ExpertGroups::kRouted;
-            const int r = mmq(part);
-            if (r <= 0) return r < 0 ? mmq(grp) : r;
+            const int r = mmq(part, UINT32_MAX);
+            if (r <= 0) return r;
             part.which = ExpertGroups::kShared;
             return tile(part, grp.n_shared);
         }
-        return mmq(grp);
+        return mmq(grp, UINT32_MAX);
     } else {
-        const int r = mmq(grp);
-        return r < 0 && (quant == PULSAR_QUANT_Q3_K || quant == PULSAR_QUANT_IQ4_XS) ? tile(grp, n_group) : r;
+        auto tile = [&](uint32_t b) {
+            return launch_tile_csr(pair, quant, out, grp, weights, act, k_dim, n_rows, n_used, n_group, row_bytes,
+                                   act_op, b);
+        };
+        if (n_group > 1024u) return mmq(grp, UINT32_MAX);  // more than the tile's blocks count
+        const int r = mmq(grp, bound);
+        if (r < 0) return quant == PULSAR_QUANT_Q3_K || quant == PULSAR_QUANT_IQ4_XS ? tile(0u) : r;
+        return r == 0 ? r : tile(bound);
     }
 }
 

@@ -5,50 +5,29 @@
 
 namespace pk {
 
-// Grouped expert stages: block = (row block, expert group), the group's
-// (token, slot) pairs in tiles of 16 NS. PAIR: row tile 0 of a wave is 16 gate
-// rows, row tile 1 the same rows of up, so a lane ends with both values of a
-// (row, pair) and applies the combine itself.
-template <uint32_t Q, bool PAIR, uint32_t WR, uint32_t WK, uint32_t NS, typename G>
-__global__ __launch_bounds__(256, 2) void tile_grouped_kernel(float *__restrict__ out, const G src,
-                                                              const float *__restrict__ weights,
-                                                              const pulsar_block_q8_K *__restrict__ act, uint32_t nb,
-                                                              uint32_t n_rows, uint32_t n_used, uint64_t row_bytes,
-                                                              uint32_t act_op, uint32_t min_pairs) {
-    using T = Tile<Q, WR, WK, NS>;
-    constexpr uint32_t kRows = PAIR ? 16u * WR : 32u * WR;
-    __shared__ __align__(16) uint8_t buf0[T::kBuf];
-    __shared__ __align__(16) uint8_t buf1[T::kBuf];
-    __shared__ uint32_t pr_l[T::kTok];
-    extern __shared__ uint32_t lst[];
-    const typename G::Group grp = src.group(blockIdx.y);
-    const pulsar_expert_ptrs &p = grp.p;
-    const uint8_t *m0 = (const uint8_t *)(PAIR ? p.gate : p.down), *m1 = (const uint8_t *)(PAIR ? p.up : p.down);
-    const bool nul = grp.is_null();  // block-uniform, as every exit below
-    if (!nul && (!m0 || !m1)) return;
-    uint32_t s0, s1;
-    src.range_block(grp, lst, s0, s1);
-    // with a bound the other kernel takes the shorter groups and the NULL one
-    if (s0 >= s1 || s1 - s0 < min_pairs || (nul && min_pairs != 0u)) return;
-    const uint32_t rb = blockIdx.x * kRows;
-    if (nul) {  // unrouted slots: their rows of this block are 0
-        for (uint32_t it = threadIdx.x; it < (s1 - s0) * kRows; it += 256u) {
-            const uint32_t pr = src.pair(s0 + it / kRows, lst), row = rb + it % kRows;
-            if (row < n_rows) out[((uint64_t)(pr >> 4) * n_used + (pr & 15u)) * n_rows + row] = 0.0f;
-        }
-        return;
-    }
-    PK_FMT_LUT(Q)
-    const uint32_t lane = threadIdx.x & 63u, i = lane & 15u, q = lane >> 4, wave = threadIdx.x >> 6;
-    const uint32_t row0 = rb + (PAIR ? 16u : 32u) * (wave % WR) + i, row1 = PAIR ? row0 : row0 + 16u;
-    const uint8_t *w0 = as_global(m0) + (uint64_t)(row0 < n_rows ? row0 : n_rows - 1u) * row_bytes;
-    const uint8_t *w1 = as_global(m1) + (uint64_t)(row1 < n_rows ? row1 : n_rows - 1u) * row_bytes;
-    const float gb = PAIR && p.gate_b && row0 < n_rows ? ldwf(p.gate_b + row0) : 0.0f;
-    const float ub = PAIR && p.up_b && row0 < n_rows ? ldwf(p.up_b + row0) : 0.0f;
-    for (uint32_t t0 = s0; t0 < s1; t0 += T::kTok) {
-        const uint32_t np = s1 - t0 < T::kTok ? s1 - t0 : T::kTok;
-        if (t0 != s0) __syncthreads();  // the previous tile's pairs are stored
-        if (threadIdx.x < np) pr_l[threadIdx.x] = src.pair(t0 + threadIdx.x, lst);
+// One pair tile of a group: rows [rb, rb + kRows) of expert p times the np
+// pairs that pair(t) gives. PAIR: row tile 0 of a wave is 16 gate rows, row
+// tile 1 the same rows of up, so a lane ends with both values of a (row, pair)
+// and applies the combine itself.
+template <uint32_t Q, bool PAIR, uint32_t NS>
+struct GroupTile {
+    using T = Tile<Q, 4, 1, NS>;
+    static constexpr uint32_t kRows = PAIR ? 64u : 128u;
+
+    template <typename PairOf>
+    PK_DEV static void run(uint8_t *buf0, uint8_t *buf1, const uint2 *lut, uint32_t *pr_l, float *out,
+                           const pulsar_expert_ptrs &p, const float *weights, const pulsar_block_q8_K *act, uint32_t nb,
+                           uint32_t n_rows, uint32_t n_used, uint64_t row_bytes, uint32_t act_op, uint32_t rb,
+                           uint32_t np, PairOf pair_of) {
+        const uint32_t lane = threadIdx.x & 63u, i = lane & 15u, q = lane >> 4, wave = threadIdx.x >> 6;
+        const uint32_t row0 = rb + (PAIR ? 16u : 32u) * wave + i, row1 = PAIR ? row0 : row0 + 16u;
+        const uint8_t *m0 = (const uint8_t *)(PAIR ? p.gate : p.down), *m1 = (const uint8_t *)(PAIR ? p.up : p.down);
+        const uint8_t *w0 = as_global(m0) + (uint64_t)(row0 < n_rows ? row0 : n_rows - 1u) * row_bytes;
+        const uint8_t *w1 = as_global(m1) + (uint64_t)(row1 < n_rows ? row1 : n_rows - 1u) * row_bytes;
+        const float gb = PAIR && p.gate_b && row0 < n_rows ? ldwf(p.gate_b + row0) : 0.0f;
+        const float ub = PAIR && p.up_b && row0 < n_rows ? ldwf(p.up_b + row0) : 0.0f;
+        __syncthreads();  // the previous tile's pairs are stored
+        if (threadIdx.x < np) pr_l[threadIdx.x] = pair_of(threadIdx.x);
         __syncthreads();
         T tile;
         auto off = [&](uint32_t t) {
@@ -63,7 +42,7 @@ __global__ __launch_bounds__(256, 2) void tile_grouped_kernel(float *__restrict_
 #pragma unroll
                 for (uint32_t r = 0; r < 4; r++) {
                     const uint32_t t = 16u * n + 4u * q + r;
-                    if (!T::mine(n, r, wave / WR) || t >= np) continue;
+                    if (t >= np) continue;
                     const uint32_t pr = pr_l[t];
                     const uint64_t so = (uint64_t)(pr >> 4) * n_used + (pr & 15u);
                     float *o = out + so * n_rows;
@@ -78,14 +57,116 @@ __global__ __launch_bounds__(256, 2) void tile_grouped_kernel(float *__restrict_
                     }
                 }
         };
-        if (NS > 1u && np <= 16u)
+        // the 16-token slices that hold pairs
+        if (np <= 16u)
             part(std::integral_constant<uint32_t, 1>{});
-        else if (NS > 2u && np <= 32u)
-            part(std::integral_constant<uint32_t, NS < 2u ? 1u : 2u>{});
+        else if (np <= 32u)
+            part(std::integral_constant<uint32_t, 2>{});
         else if (NS > 4u && np <= 64u)
-            part(std::integral_constant<uint32_t, NS < 4u ? 1u : 4u>{});
+            part(std::integral_constant<uint32_t, 4>{});
         else
             part(std::integral_constant<uint32_t, NS>{});
+    }
+};
+
+// Groups found from the router's ids: block = (row block, group), the group's
+// pairs in tiles of 16 NS one after the other.
+template <uint32_t Q, bool PAIR, uint32_t NS>
+__global__ __launch_bounds__(256, 2) void tile_experts_kernel(float *__restrict__ out, const ExpertGroups src,
+                                                              const float *__restrict__ weights,
+                                                              const pulsar_block_q8_K *__restrict__ act, uint32_t nb,
+                                                              uint32_t n_rows, uint32_t n_used, uint64_t row_bytes,
+                                                              uint32_t act_op) {
+    using GT = GroupTile<Q, PAIR, NS>;
+    __shared__ __align__(16) uint8_t buf0[GT::T::kBuf];
+    __shared__ __align__(16) uint8_t buf1[GT::T::kBuf];
+    __shared__ uint32_t pr_l[GT::T::kTok];
+    extern __shared__ uint32_t lst[];
+    const ExpertGroups::Group grp = src.group(blockIdx.y);
+    const pulsar_expert_ptrs &p = grp.p;
+    const bool nul = grp.is_null();  // block-uniform, as every exit below
+    if (!nul && !(PAIR ? p.gate && p.up : p.down != nullptr)) return;
+    uint32_t s0, s1;
+    src.range_block(grp, lst, s0, s1);
+    if (s0 >= s1) return;
+    const uint32_t rb = blockIdx.x * GT::kRows;
+    if (nul) {  // unrouted slots: their rows of this block are 0
+        for (uint32_t it = threadIdx.x; it < (s1 - s0) * GT::kRows; it += 256u) {
+            const uint32_t pr = lst[s0 + it / GT::kRows], row = rb + it % GT::kRows;
+            if (row < n_rows) out[((uint64_t)(pr >> 4) * n_used + (pr & 15u)) * n_rows + row] = 0.0f;
+        }
+        return;
+    }
+    PK_FMT_LUT(Q)
+    for (uint32_t t0 = s0; t0 < s1; t0 += GT::T::kTok)
+        GT::run(buf0, buf1, lut, pr_l, out, p, weights, act, nb, n_rows, n_used, row_bytes, act_op, rb,
+                s1 - t0 < GT::T::kTok ? s1 - t0 : GT::T::kTok, [&](uint32_t t) { return lst[t0 + t]; });
+}
+
+constexpr uint32_t kCsrGroups = 1024;  // groups whose tile counts a block keeps
+
+// A caller's CSR, whose group sizes only the device knows. A launch of at most
+// kTileSlots blocks: each counts the tiles of every group (one round trip),
+// and block b takes the (tile, row block) items b, b + grid, ...: uneven groups
+// spread evenly, and where the groups are short (fewer than bound / 4 pairs on
+// average: mmq.hip's kernel, launched before, has taken them) the blocks end
+// after one load.
+template <uint32_t Q, bool PAIR, uint32_t NS>
+__global__ __launch_bounds__(256, 2) void tile_csr_kernel(float *__restrict__ out, const CsrGroups src,
+                                                          const float *__restrict__ weights,
+                                                          const pulsar_block_q8_K *__restrict__ act, uint32_t nb,
+                                                          uint32_t n_rows, uint32_t n_used, uint64_t row_bytes,
+                                                          uint32_t act_op, uint32_t n_group, uint32_t bound) {
+    using GT = GroupTile<Q, PAIR, NS>;
+    constexpr uint32_t kTok = GT::T::kTok;
+    if (4ull * (src.starts[n_group] - src.starts[0]) < (uint64_t)bound * n_group) return;
+    __shared__ __align__(16) uint8_t buf0[GT::T::kBuf];
+    __shared__ __align__(16) uint8_t buf1[GT::T::kBuf];
+    __shared__ uint32_t pr_l[kTok];
+    __shared__ uint32_t first[kCsrGroups + 1u];  // tiles before group g
+    __shared__ uint32_t wsum[4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    uint32_t n[4], sum = 0u;  // groups 4 tid .. 4 tid + 3
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; k++) {
+        const uint32_t g = 4u * tid + k;
+        const uint32_t b = src.starts[g < n_group ? g : n_group], e = src.starts[g < n_group ? g + 1u : n_group];
+        n[k] = e > b ? (e - b + kTok - 1u) / kTok : 0u;
+        sum += n[k];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (uint32_t d = 1; d < 64u; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)incl, d, 64);
+        incl += lane >= d ? o : 0u;
+    }
+    if (lane == 63u) wsum[wave] = incl;
+    __syncthreads();
+    uint32_t at = incl - sum;
+#pragma unroll
+    for (uint32_t w = 0; w < 3u; w++) at += w < wave ? wsum[w] : 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; k++) {
+        first[4u * tid + k] = at;
+        at += n[k];
+    }
+    if (tid == 255u) first[kCsrGroups] = at;
+    PK_FMT_LUT(Q)
+    __syncthreads();
+    const uint32_t n_rb = (n_rows + GT::kRows - 1u) / GT::kRows;
+    const uint64_t total = (uint64_t)first[kCsrGroups] * n_rb;
+    for (uint64_t item = blockIdx.x; item < total; item += gridDim.x) {
+        const uint32_t tl = (uint32_t)(item / n_rb), rb = (uint32_t)(item % n_rb) * GT::kRows;
+        uint32_t g = 0u;  // the last group with first[g] <= tl
+#pragma unroll
+        for (uint32_t s = kCsrGroups / 2u; s != 0u; s >>= 1)
+            if (first[g + s] <= tl) g += s;
+        g = (uint32_t)__builtin_amdgcn_readfirstlane((int)g);
+        const pulsar_expert_ptrs p = src.gptrs[g];
+        if (!(PAIR ? p.gate && p.up : p.down != nullptr)) continue;  // block-uniform
+        const uint32_t t0 = src.starts[g] + (tl - first[g]) * kTok, t1 = src.starts[g + 1u];
+        GT::run(buf0, buf1, lut, pr_l, out, p, weights, act, nb, n_rows, n_used, row_bytes, act_op, rb,
+                t1 - t0 < kTok ? t1 - t0 : kTok, [&](uint32_t t) { return src.pairs[t0 + t]; });
     }
 }
 
@@ -113,51 +194,56 @@ uint32_t tile_min_quarter_pairs(bool pair, uint32_t quant) {
     }
 }
 
-template <uint32_t Q, bool PAIR, typename G>
-static int launch_tile_grouped_q(float *out, const G &src, const float *weights, const pulsar_block_q8_K *act,
-                                 uint32_t nb, uint32_t n_rows, uint32_t n_used, uint32_t n_group, uint64_t row_bytes,
-                                 uint32_t act_op, uint32_t lst_bytes, uint32_t min_pairs) {
-    // 64-pair tiles; 128 where a caller's CSR may hold long groups and the
-    // format's registers allow it (Q2_K gate / up, 96 pairs: 685 -> 562 us,
-    // 16 pairs 240 / 235; Q4_K spills: 279 -> 319)
-    constexpr uint32_t NS = std::is_same<G, CsrGroups>::value && Q != PULSAR_QUANT_Q4_K && Q != PULSAR_QUANT_Q5_K ? 8 : 4;
-    constexpr uint32_t kRows = PAIR ? 64u : 128u;
-    hipLaunchKernelGGL((tile_grouped_kernel<Q, PAIR, 4, 1, NS, G>), dim3((n_rows + kRows - 1u) / kRows, n_group),
-                       dim3(256), lst_bytes, pk::stream(), out, src, weights, act, nb, n_rows, n_used, row_bytes,
-                       act_op, min_pairs);
-    return launch_ok(PAIR ? "moe pair swiglu grouped (tile) launch" : "moe down grouped (tile) launch");
-}
+#define PK_TILE_FORMATS(F)                                                                                            \
+    F(PULSAR_QUANT_Q4_K) F(PULSAR_QUANT_Q5_K) F(PULSAR_QUANT_Q6_K) F(PULSAR_QUANT_Q2_K) F(PULSAR_QUANT_Q3_K)          \
+    F(PULSAR_QUANT_IQ4_XS) F(PULSAR_QUANT_IQ2_XXS)
 
-// The grouped stages on the tile, for the groups of at least min_pairs pairs.
-template <typename G>
-int launch_tile_grouped(bool pair, uint32_t quant, float *out, const G &src, const float *weights,
+// The grouped stages of an ExpertGroups source on the tile, n_group groups.
+int launch_tile_experts(bool pair, uint32_t quant, float *out, const ExpertGroups &src, const float *weights,
                         const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
-                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
-                        uint32_t min_pairs) {
-    const uint32_t nb = k_dim / 256u;
-#define PK_TG(Q)                                                                                                     \
-    case Q:                                                                                                          \
-        return pair ? launch_tile_grouped_q<Q, true, G>(out, src, weights, act, nb, n_rows, n_used, n_group, row_bytes, \
-                                                        act_op, lst_bytes, min_pairs)                                \
-                    : launch_tile_grouped_q<Q, false, G>(out, src, weights, act, nb, n_rows, n_used, n_group,          \
-                                                         row_bytes, act_op, lst_bytes, min_pairs);
+                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes) {
+#define PK_LAUNCH(Q, P)                                                                                               \
+    hipLaunchKernelGGL((tile_experts_kernel<Q, P, 4>),                                                                \
+                       dim3((n_rows + GroupTile<Q, P, 4>::kRows - 1u) / GroupTile<Q, P, 4>::kRows, n_group), dim3(256), \
+                       lst_bytes, pk::stream(), out, src, weights, act, k_dim / 256u, n_rows, n_used, row_bytes, act_op)
+#define PK_CASE(Q)                  \
+    case Q:                         \
+        if (pair)                   \
+            PK_LAUNCH(Q, true);     \
+        else                        \
+            PK_LAUNCH(Q, false);    \
+        break;
     switch (quant) {
-        PK_TG(PULSAR_QUANT_Q4_K)
-        PK_TG(PULSAR_QUANT_Q5_K)
-        PK_TG(PULSAR_QUANT_Q6_K)
-        PK_TG(PULSAR_QUANT_Q2_K)
-        PK_TG(PULSAR_QUANT_Q3_K)
-        PK_TG(PULSAR_QUANT_IQ4_XS)
-        PK_TG(PULSAR_QUANT_IQ2_XXS)
+        PK_TILE_FORMATS(PK_CASE)
     default: return reject("grouped tile (quant)");
     }
-#undef PK_TG
+#undef PK_LAUNCH
+    return launch_ok(pair ? "moe pair swiglu experts (tile) launch" : "moe down experts (tile) launch");
 }
-template int launch_tile_grouped<CsrGroups>(bool, uint32_t, float *, const CsrGroups &, const float *,
-                                            const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t, uint32_t,
-                                            uint64_t, uint32_t, uint32_t, uint32_t);
-template int launch_tile_grouped<ExpertGroups>(bool, uint32_t, float *, const ExpertGroups &, const float *,
-                                               const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t, uint32_t,
-                                               uint64_t, uint32_t, uint32_t, uint32_t);
+
+// The grouped stages of a caller's CSR on the tile, where the groups have bound
+// / 4 pairs or more on average (0: in any case). 128-pair tiles where the
+// format's registers allow it (Q2_K gate / up, 96 pairs per group: 685 -> 562
+// us, 16 pairs 240 / 235; Q4_K spills: 279 -> 319).
+int launch_tile_csr(bool pair, uint32_t quant, float *out, const CsrGroups &src, const float *weights,
+                    const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used, uint32_t n_group,
+                    uint64_t row_bytes, uint32_t act_op, uint32_t bound) {
+#define PK_LAUNCH(Q, P)                                                                                              \
+    do {                                                                                                             \
+        constexpr uint32_t NS = Q == PULSAR_QUANT_Q4_K || Q == PULSAR_QUANT_Q5_K ? 4 : 8;                            \
+        const uint64_t rbs = (n_rows + GroupTile<Q, P, NS>::kRows - 1u) / GroupTile<Q, P, NS>::kRows;                \
+        const uint64_t most = rbs * n_group;                                                                         \
+        hipLaunchKernelGGL((tile_csr_kernel<Q, P, NS>), dim3((uint32_t)(most < 512u ? most : 512u)), dim3(256), 0,   \
+                           pk::stream(), out, src, weights, act, k_dim / 256u, n_rows, n_used, row_bytes, act_op,    \
+                           n_group, bound);                                                                          \
+    } while (0)
+    switch (quant) {
+        PK_TILE_FORMATS(PK_CASE)
+    default: return reject("grouped tile (quant)");
+    }
+#undef PK_CASE
+#undef PK_LAUNCH
+    return launch_ok(pair ? "moe pair swiglu grouped (tile) launch" : "moe down grouped (tile) launch");
+}
 
 }  // namespace pk
