@@ -91,6 +91,18 @@ struct TileW {
 template <uint32_t Q>
 struct TileFmt;
 
+// The words of a Raw as values the compiler must have in registers here: its
+// loads cannot be moved past this point, to where the words are decoded.
+template <typename Raw>
+PK_DEV void hold_raw(Raw &r) {
+    struct Words {
+        uint32_t v[sizeof(Raw) / 4u];
+    } w = __builtin_bit_cast(Words, r);
+#pragma unroll
+    for (uint32_t k = 0; k < sizeof(Raw) / 4u; k++) asm volatile("" : "+v"(w.v[k]));
+    r = __builtin_bit_cast(Raw, w);
+}
+
 // the 6-bit scales and mins of the Q4_K / Q5_K header (cpu_dot.rs:147-156), a
 // byte each
 struct KqScales {
@@ -431,9 +443,9 @@ struct Tile {
 
     // w0, w1: the lane's two weight rows; xb + off_of(t): the q8_K row of token
     // t < np (0 < np <= kTok); buf0, buf1: kBuf bytes each, two distinct LDS
-    // arrays. NC: the token slices computed (16 NC >= np). On return the lanes
+    // arrays. On return the lanes
     // of wave (wr, wk) hold the sums of their share of the elements (mine()).
-    template <uint32_t NC = NS, typename OffOf>
+    template <typename OffOf>
     PK_DEV void run(uint8_t *buf0, uint8_t *buf1, const uint2 *lut, const uint8_t *w0, const uint8_t *w1, uint32_t nb,
                     uint32_t np, const uint8_t *xb, OffOf off_of) {
         const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -526,8 +538,8 @@ struct Tile {
             v4i_t pl[2], ph[2];
             read_a(0u);
 #pragma unroll
-            for (uint32_t n = 0; n < NC; n++) {
-                if (n + 1u < NC) read_a(n + 1u);
+            for (uint32_t n = 0; n < NS; n++) {
+                if (n + 1u < NS) read_a(n + 1u);
                 v4i_t dl[2] = {}, dh[2] = {};
 #pragma unroll
                 for (uint32_t s = 0; s < 4; s++)
@@ -543,7 +555,7 @@ struct Tile {
                     ph[rt] = dh[rt];
                 }
             }
-            finish(NC - 1u, pl, ph);
+            finish(NS - 1u, pl, ph);
             arrived();
         };
         arrived();
@@ -560,13 +572,13 @@ struct Tile {
                 return (float *)(wv < 2u ? buf0 : buf1) + (((wv & 1u) * NS + n) * 8u + rt * 4u + r) * 64u + lane;
             };
 #pragma unroll
-            for (uint32_t n = 0; n < NC; n++)
+            for (uint32_t n = 0; n < NS; n++)
 #pragma unroll
                 for (uint32_t e = 0; e < 8; e++) *part(wave, n, e >> 2, e & 3u) = acc[n][e >> 2][e & 3u];
             __syncthreads();
             const uint32_t wr = wave % WR;
 #pragma unroll
-            for (uint32_t n = 0; n < NC; n++)
+            for (uint32_t n = 0; n < NS; n++)
 #pragma unroll
                 for (uint32_t e = 0; e < 8; e++)
                     if (mine(n, e & 3u, wk)) {
@@ -581,6 +593,160 @@ struct Tile {
     // Which K slice finishes element r of slice n (both row tiles): the 4 NS
     // (slice, element) places in WK runs
     PK_DEV static bool mine(uint32_t n, uint32_t r, uint32_t wk) { return WK == 1u || (4u * n + r) * WK / (4u * NS) == wk; }
+};
+
+// The tile of the expert groups: Tile<Q, 4, 1, NS> with the order of a token
+// slice's steps fixed. Its time goes to LDS reads that are waited for at once:
+// at 250 registers the compiler reads a step's tokens right before their MFMAs
+// (timed without those reads, a Q4_K tile of 8 slices takes 51 us instead of
+// 72). Here the tokens of a step are read again, for the next slice, as soon as
+// the step's MFMAs are issued, 12 MFMAs ahead of their use and into the same
+// registers, with a quarter of the previous slice's fp32 step beside them.
+// The lane keeps the 32-bit q8_K rows of the records it copies and forms their
+// addresses, two registers each, in every iteration: half the spills. Prefill
+// of 128 Q4_K / Q6_K experts, 1536 tokens top-8: 437 -> 401 us a layer; IQ2_XXS
+// chunk of 100 tokens: 498 -> 485. The dense kernel keeps Tile::run: fixed in
+// this order its 8-slice Q4_K tile spills 37 registers (77 -> 91 us), and its
+// tiles of 2 to 4 slices take 1-2% longer.
+template <uint32_t Q, uint32_t NS>
+struct GroupedTile : Tile<Q, 4, 1, NS> {
+    using T = Tile<Q, 4, 1, NS>;
+    using F = TileFmt<Q>;
+
+    // As Tile::run, with row_of(t): the q8_K row, of nb blocks each from xb on,
+    // of token t. NC: the token slices computed (16 NC >= np).
+    template <uint32_t NC, typename RowOf>
+    PK_DEV void run(uint8_t *buf0, uint8_t *buf1, const uint2 *lut, const uint8_t *w0, const uint8_t *w1, uint32_t nb,
+                    uint32_t np, const uint8_t *xb, RowOf row_of) {
+        const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const uint32_t i = lane & 15u, q = lane >> 4;
+        // tokens past np: the last one again
+        auto row = [&](uint32_t t) { return row_of(t < np ? t : np - 1u); };
+        uint32_t xrow[NS];
+#pragma unroll
+        for (uint32_t m = 0; m < NS; m++) xrow[m] = row(4u * (wave + 4u * m) + lane / 16u);
+        const uint32_t bs_blk = T::kRec >= 128u ? wave : wave % (T::kRec / 32u), d_blk = wave % (T::kRec / 64u);
+        const uint32_t bs_row = row(32u * bs_blk + lane / 2u), d_row = row(64u * d_blk + lane);
+        // as Tile::run's copies
+        auto dma = [&](uint8_t *buf, uint32_t it) {
+            uint32_t stride = nb * 292u;
+            asm volatile("" : "+s"(stride));  // the products are not hoisted out of the loop
+            auto src = [&](uint32_t r, uint32_t at) {
+                return (const PK_GLOBAL uint32_t *)(xb + ((it < nb ? it : nb - 1u) * 292u + at) + (uint64_t)r * stride);
+            };
+#pragma unroll
+            for (uint32_t m = 0; m < NS; m++) {
+                const uint32_t r0 = 4u * (wave + 4u * m), rec = r0 + lane / 16u;
+                __builtin_amdgcn_global_load_lds(src(xrow[m], 4u + 16u * ((lane ^ rec) & 15u)),
+                                                 (PK_LDS uint32_t *)(buf + r0 * 256u), 16, 0, 0);
+            }
+            if (F::kMin)
+                __builtin_amdgcn_global_load_lds(src(bs_row, 260u + 16u * (lane & 1u)),
+                                                 (PK_LDS uint32_t *)(buf + T::kBsum + 1024u * bs_blk), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(src(d_row, 0u), (PK_LDS uint32_t *)(buf + T::kD + 256u * d_blk), 4, 0, 0);
+        };
+#pragma unroll
+        for (uint32_t n = 0; n < NS; n++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) this->acc[n][0][r] = this->acc[n][1][r] = 0.0f;
+        uint32_t ao[4];  // byte offset of the lane's piece of step s, token slice 0
+#pragma unroll
+        for (uint32_t s = 0; s < 4; s++) ao[s] = i * 256u + 16u * (F::piece(s, q) ^ i);
+        dma(buf0, 0u);
+        typename F::Raw raw[2];
+        auto load_w = [&](uint32_t it) {  // past the end: the last super-block again
+            const uint64_t o = (uint64_t)(it < nb ? it : nb - 1u) * F::kSb;
+            raw[0] = F::load(w0 + o, q);
+            raw[1] = F::load(w1 + o, q);
+        };
+        load_w(0u);
+        auto arrived = [] {
+            __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the wave's DMA writes are in LDS
+            __syncthreads();
+        };
+        auto step = [&](const uint8_t *buf, uint8_t *nbuf, uint32_t it) {
+            TileW tw[2];
+            F::decode(raw[0], q, lut, tw[0]);
+            F::decode(raw[1], q, lut, tw[1]);
+            __builtin_amdgcn_sched_barrier(0);
+            dma(nbuf, it + 1u);
+            // late where the accumulators leave few registers
+            constexpr uint32_t kLoadAt = NC > 4u ? NC - 2u : 0u;
+            if (kLoadAt == 0u) load_w(it + 1u);
+            __builtin_amdgcn_sched_barrier(0);
+            uint4 a[4];
+            auto read_a = [&](uint32_t n, uint32_t s) { a[s] = *(const uint4 *)(buf + ao[s] + 4096u * n); };
+            // what the fp32 step of a slice needs besides its integer sums
+            struct Side {
+                uint4 y;
+                uint2 b;
+                v4f_t ms[2];
+            };
+            auto read_side = [&](uint32_t n, Side &d) {
+                d.y = *(const uint4 *)(buf + T::kD + (16u * n + 4u * q) * 4u);
+                if constexpr (F::kMin) d.b = *(const uint2 *)(buf + T::kBsum + (16u * n + i) * 32u + 8u * q);
+            };
+            auto min_terms = [&](Side &d) {
+                if constexpr (F::kMin) {
+                    const uint2 bh = make_uint2(f16_of_i16(d.b.x), f16_of_i16(d.b.y));
+                    d.ms[0] = mfma16_f16(bh, tw[0].mins);
+                    d.ms[1] = mfma16_f16(bh, tw[1].mins);
+                }
+            };
+            // the fp32 step of token 4q + r of slice n
+            auto finish = [&](uint32_t n, uint32_t r, const Side &d, const v4i_t (&dl)[2], const v4i_t (&dh)[2]) {
+                const float yd = __uint_as_float(word4(d.y, r));
+#pragma unroll
+                for (int rt = 0; rt < 2; rt++) {
+                    const int32_t sum = F::kHi ? (int32_t)((uint32_t)dh[rt][r] << F::kShift) + dl[rt][r] : dl[rt][r];
+                    float v = (F::kNeg ? -tw[rt].xd : tw[rt].xd) * (float)sum;
+                    if (F::kMin) v = __builtin_fmaf(-tw[rt].xmin, d.ms[rt][r], v);
+                    this->acc[n][rt][r] = __builtin_fmaf(yd, v, this->acc[n][rt][r]);
+                }
+            };
+            v4i_t pl[2], ph[2];
+            Side ps;
+#pragma unroll
+            for (uint32_t s = 0; s < 4; s++) read_a(0u, s);
+#pragma unroll
+            for (uint32_t n = 0; n < NC; n++) {
+                v4i_t dl[2] = {}, dh[2] = {};
+                Side d;
+                read_side(n, d);
+                if (n > 0u && n == kLoadAt) load_w(it + 1u);
+#pragma unroll
+                for (uint32_t s = 0; s < 4; s++) {
+#pragma unroll
+                    for (int rt = 0; rt < 2; rt++) {
+                        dl[rt] = mfma64(a[s], tw[rt].lo[s], dl[rt]);
+                        if (F::kHi) dh[rt] = mfma64(a[s], tw[rt].hi[s], dh[rt]);
+                    }
+                    if (n + 1u < NC) read_a(n + 1u, s);
+                    if (n > 0u) finish(n - 1u, s, ps, pl, ph);
+                    if (s == 3u) min_terms(d);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int rt = 0; rt < 2; rt++) {
+                    pl[rt] = dl[rt];
+                    ph[rt] = dh[rt];
+                }
+                ps = d;
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) finish(NC - 1u, r, ps, pl, ph);
+            arrived();
+            hold_raw(raw[0]);
+            hold_raw(raw[1]);
+        };
+        arrived();
+        for (uint32_t it = 0;;) {
+            step(buf0, buf1, it);
+            if (++it == nb) break;
+            step(buf1, buf0, it);
+            if (++it == nb) break;
+        }
+    }
 };
 
 }  // namespace pk

@@ -11,7 +11,7 @@ namespace pk {
 // and applies the combine itself.
 template <uint32_t Q, bool PAIR, uint32_t NS>
 struct GroupTile {
-    using T = Tile<Q, 4, 1, NS>;
+    using T = GroupedTile<Q, NS>;
     static constexpr uint32_t kRows = PAIR ? 64u : 128u;
 
     template <typename PairOf>
@@ -30,13 +30,13 @@ struct GroupTile {
         if (threadIdx.x < np) pr_l[threadIdx.x] = pair_of(threadIdx.x);
         __syncthreads();
         T tile;
-        auto off = [&](uint32_t t) {
+        auto row = [&](uint32_t t) {
             const uint32_t pr = pr_l[t];
-            return (uint64_t)(PAIR ? pr >> 4 : (pr >> 4) * n_used + (pr & 15u)) * (nb * 292u);
+            return PAIR ? pr >> 4 : (pr >> 4) * n_used + (pr & 15u);
         };
         auto part = [&](auto nc) {
             constexpr uint32_t NC = decltype(nc)::value;
-            tile.template run<NC>(buf0, buf1, lut, w0, w1, nb, np, (const uint8_t *)act, off);
+            tile.template run<NC>(buf0, buf1, lut, w0, w1, nb, np, (const uint8_t *)act, row);
 #pragma unroll
             for (uint32_t n = 0; n < NC; n++)
 #pragma unroll
