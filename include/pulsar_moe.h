@@ -266,11 +266,14 @@ int pulsar_moe_route(void *selected, void *weights, void *ptrs, void *slot_weigh
  * instead of a CSR (no reference counterpart: the reference groups on the
  * host, crates/engine/src/lib.rs:8357-8392). Each routed (token, slot)
  * pair runs in the group of its expert, shared slot i (s = k_used + i,
- * weight 1) of every token in a group of its own, as
+ * weight 1) of every token in a group of its own, exactly as
  * pulsar_moe_pair_swiglu_grouped / pulsar_moe_down_grouped would for the
- * same pairs: the same exact integer sums, and the same rows bit for bit
- * wherever both choose the same kernel by the groups' mean size (else their
- * fp32 steps round differently in the last bits).
+ * same pairs, so the rows they write are bit-identical to those calls',
+ * whatever the sizes of the groups. One exception: stages that the lane
+ * kernels run where groups are short (Q3_K, IQ4_XS; rows too wide for the
+ * 16-row kernel's staged activations) equal them bit for bit where both
+ * calls' groups have the same mean size (else their super-blocks are added
+ * in another order).
  * Slots whose id is outside [0, n_expert) get rows of 0 in mid (partial),
  * so every row of mid [n_tok][k_used + n_shared][mid_dim] (partial
  * [..][out_dim]) is written and partial needs no zeroing. slot_weights

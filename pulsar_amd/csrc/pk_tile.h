@@ -605,7 +605,9 @@ struct Tile {
 // The lane keeps the 32-bit q8_K rows of the records it copies and forms their
 // addresses, two registers each, in every iteration: half the spills. Prefill
 // of 128 Q4_K / Q6_K experts, 1536 tokens top-8: 437 -> 401 us a layer; IQ2_XXS
-// chunk of 100 tokens: 498 -> 485. The dense kernel keeps Tile::run: fixed in
+// chunk of 100 tokens: 498 -> 485. The 16-row kernel's fp32 step, which has three
+// more vector operations for formats with mins, takes that layer from 397 to
+// 404. The dense kernel keeps Tile::run: fixed in
 // this order its 8-slice Q4_K tile spills 37 registers (77 -> 91 us), and its
 // tiles of 2 to 4 slices take 1-2% longer.
 template <uint32_t Q, uint32_t NS>
@@ -693,15 +695,20 @@ struct GroupedTile : Tile<Q, 4, 1, NS> {
                     d.ms[1] = mfma16_f16(bh, tw[1].mins);
                 }
             };
-            // the fp32 step of token 4q + r of slice n
+            // the fp32 step of token 4q + r of slice n, with the products and
+            // roundings of the 16-row kernel (mmq.hip): the integer sums are
+            // exact in both, so a pair's value is the same whichever runs it
             auto finish = [&](uint32_t n, uint32_t r, const Side &d, const v4i_t (&dl)[2], const v4i_t (&dh)[2]) {
                 const float yd = __uint_as_float(word4(d.y, r));
 #pragma unroll
                 for (int rt = 0; rt < 2; rt++) {
                     const int32_t sum = F::kHi ? (int32_t)((uint32_t)dh[rt][r] << F::kShift) + dl[rt][r] : dl[rt][r];
-                    float v = (F::kNeg ? -tw[rt].xd : tw[rt].xd) * (float)sum;
-                    if (F::kMin) v = __builtin_fmaf(-tw[rt].xmin, d.ms[rt][r], v);
-                    this->acc[n][rt][r] = __builtin_fmaf(yd, v, this->acc[n][rt][r]);
+                    const float xy = (F::kNeg ? -tw[rt].xd : tw[rt].xd) * yd;
+                    float &a = this->acc[n][rt][r];
+                    if constexpr (F::kMin)
+                        a += xy * (float)sum - tw[rt].xmin * yd * d.ms[rt][r];
+                    else
+                        a = __builtin_fmaf(xy, (float)sum, a);
                 }
             };
             v4i_t pl[2], ph[2];

@@ -1,0 +1,94 @@
+"""Which kernel a grouped expert stage runs on, and that its rows do not show it:
+the 16-row kernel (csrc/mmq.hip), the wide tile (csrc/tile_moe.hip) and the lane
+kernels (csrc/moe.hip) take a stage by the size of its groups, so every case here
+puts the same pairs on two sides of a choice or checks one side on the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from pulsar_amd import formats as fm
+from pulsar_amd import kernels as K
+from pulsar_amd.formats import QUANT_IQ2_XXS, QUANT_Q2_K, QUANT_Q4_K, QUANT_Q5_K, QUANT_Q6_K, row_bytes
+from tests.gpu_util import down as down_np
+from tests.gpu_util import up
+from tests.test_gpu_tile import SIZES, check_grouped, grouped_case
+
+pytestmark = pytest.mark.gpu
+ROW16 = [QUANT_Q2_K, QUANT_IQ2_XXS, QUANT_Q4_K, QUANT_Q5_K, QUANT_Q6_K]  # formats of the 16-row kernel and the tile
+
+
+class Stage:
+    """One grouped stage over groups of the given sizes (expert e: sizes[e]
+    pairs), callable from a caller's CSR and from the router's ids."""
+
+    def __init__(self, dev, quant, down, sizes, hidden=768, ffn=330, n_used=3, seed=0):
+        rng = np.random.default_rng(seed + 2 * quant + down)
+        self.dev, self.quant, self.down, self.sizes, self.n_used = dev, quant, down, list(sizes), n_used
+        self.rows, self.cols = (hidden, ffn) if down else (ffn, hidden)
+        self.mats, self.ids, self.xq = grouped_case(quant, hidden, ffn, self.sizes, n_used, rng, down)
+        self.T, self.E, self.rb = self.ids.shape[0], len(self.sizes), row_bytes(quant, self.cols)
+        self.wts = rng.uniform(0.1, 1.0, (self.T, n_used)).astype(np.float32)
+        self.d_mats, self.d_xq, self.d_w = [up(m) for m in self.mats], up(self.xq), torch.from_numpy(self.wts).to(dev)
+        self.step = self.rows * self.rb
+
+    def entry(self, e):
+        p = [m.data_ptr() + e * self.step for m in self.d_mats]
+        return (0, 0, p[0]) if self.down else (p[0], p[1], 0)
+
+    def csr_arrays(self, order=None, pad=0, skip=0):
+        """gptrs, starts, pairs of the experts in `order` (all; -1: an empty NULL
+        group), then `pad` empty NULL groups; the listed pairs start at `skip`."""
+        order = list(range(self.E)) if order is None else list(order)
+        order += [-1] * pad
+        flat = self.ids.reshape(-1)
+        lists = [np.flatnonzero(flat == e) if e >= 0 else np.zeros(0, np.int64) for e in order]
+        g = K.expert_ptrs([self.entry(e) if e >= 0 else (0, 0, 0) for e in order])
+        i = np.concatenate(lists)
+        pairs = np.concatenate([np.zeros(skip, np.int64), i // self.n_used << 4 | i % self.n_used]).astype(np.uint32)
+        starts = (skip + np.concatenate([[0], np.cumsum([len(v) for v in lists])])).astype(np.uint32)
+        return g, starts, pairs
+
+    def run_csr(self, arrays, out=None, xq=None):
+        g, starts, pairs = (up(a) for a in arrays)
+        n_group = len(arrays[1]) - 1
+        out = torch.zeros((self.T * self.n_used, self.rows), dtype=torch.float32, device=self.dev) if out is None else out
+        xq = self.d_xq if xq is None else xq
+        if self.down:
+            K.moe_down_grouped(out, g, starts, pairs, xq, self.cols, self.rows, self.n_used, n_group, self.rb, self.quant)
+        else:
+            K.moe_pair_swiglu_grouped(out, g, starts, pairs, self.d_w, xq, self.cols, self.rows, self.n_used, n_group,
+                                      self.rb, self.quant, 0)
+        return down_np(out)
+
+    def run_experts(self, xq=None):
+        ids = self.ids.reshape(-1)
+        first = list(dict.fromkeys(int(e) for e in ids if e >= 0))
+        active = np.zeros(2 + self.E, np.uint32)
+        active[:2 + len(first)] = [len(first), int((ids == -1).sum())] + first
+        p = [m.data_ptr() for m in self.d_mats]
+        bank = (K.ExpertBank(None, None, p[0], None, None, None, 0, 0, self.step, 0, 0, 0) if self.down else
+                K.ExpertBank(p[0], p[1], None, None, None, None, self.step, self.step, 0, 0, 0, 0))
+        out = torch.full((self.T * self.n_used, self.rows), float("nan"), dtype=torch.float32, device=self.dev)
+        d_ids, d_act, xq = up(self.ids), up(active), self.d_xq if xq is None else xq
+        if self.down:
+            K.moe_down_experts(out, d_ids, d_act, xq, bank, self.E, [], self.T, self.n_used, self.cols, self.rows,
+                               self.rb, self.quant)
+        else:
+            K.moe_pair_swiglu_experts(out, d_ids, d_act, self.d_w, xq, bank, self.E, [], self.T, self.n_used,
+                                      self.cols, self.rows, self.rb, self.quant, 0)
+        return down_np(out)
+
+    def check(self, got, what):
+        check_grouped(self.quant, self.mats, self.ids, self.xq, self.wts, got, self.down, self.cols, what)
+
+
+@pytest.mark.parametrize("down", [False, True])
+@pytest.mark.parametrize("quant", ROW16, ids=lambda q: fm.NAMES[q])
+def test_rows_equal_across_kernels(dev, quant, down):
+    """The same groups from a CSR whose padding makes their mean short (the
+    16-row kernel) and from the router's ids (the tile): bit for bit equal."""
+    s = Stage(dev, quant, down, SIZES, *((330, 768) if down else (768, 330)))
+    short, tile = s.run_csr(s.csr_arrays(pad=400)), s.run_experts()
+    s.check(short, "16-row")
+    assert np.array_equal(short.view(np.uint32), tile.view(np.uint32))
+    assert np.array_equal(s.run_csr(s.csr_arrays()).view(np.uint32), tile.view(np.uint32))
