@@ -635,8 +635,11 @@ static int grouped_mfma(bool pair, uint32_t quant, float *out, const G &grp, con
                         const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
                         uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
                         const GroupSizes &sizes) {
-    // rows wider than the lane kernels take are refused for every format
-    const uint32_t bound = k_dim <= 16384u ? tile_min_quarter_pairs(pair, quant) : 0u;
+    // rows wider than the lane kernels take are refused for every format, and
+    // the tile's copies to LDS move whole dwords of act, which the other
+    // kernels load at any alignment
+    const bool fits = k_dim <= 16384u && (uintptr_t)act % 4u == 0u;
+    const uint32_t bound = fits ? tile_min_quarter_pairs(pair, quant) : 0u;
     auto mmq = [&](const G &src, uint32_t b) {
         return launch_grouped_mmq_kq(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, n_group, row_bytes,
                                      act_op, lst_bytes, b);

@@ -91,6 +91,9 @@ int launch_tile_gemm(uint32_t quant, float *out, const uint8_t *w, const pulsar_
                      uint32_t out_dim, uint32_t n_tok, uint64_t row_bytes) {
     const uint32_t nb = in_dim / 256u;
     if (nb > 65536u) return -1;  // a tile's activation offsets are 32 bits
+    // the tile's copies to LDS move whole dwords of xq, the other kernels load
+    // it at any alignment
+    if ((uintptr_t)xq % 4u != 0u) return -1;
     // Where the other kernels are at least as fast (weights from HBM, both
     // sides timed on the same matrices):
     // Q4_K, Q5_K, Q6_K have the 16-row kernel of mmq.hip, which takes chunks of

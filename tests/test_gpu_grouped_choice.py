@@ -6,12 +6,14 @@ import numpy as np
 import pytest
 import torch
 
+import oracle
 from pulsar_amd import formats as fm
 from pulsar_amd import kernels as K
+from pulsar_amd import synth
 from pulsar_amd.formats import QUANT_IQ2_XXS, QUANT_Q2_K, QUANT_Q4_K, QUANT_Q5_K, QUANT_Q6_K, row_bytes
 from tests.gpu_util import down as down_np
-from tests.gpu_util import up
-from tests.test_gpu_tile import SIZES, check_grouped, grouped_case
+from tests.gpu_util import assert_rows_close, up, zeros_f32
+from tests.test_gpu_tile import FORMATS, SIZES, check_grouped, edge_rows, grouped_case, rows_want
 
 pytestmark = pytest.mark.gpu
 ROW16 = [QUANT_Q2_K, QUANT_IQ2_XXS, QUANT_Q4_K, QUANT_Q5_K, QUANT_Q6_K]  # formats of the 16-row kernel and the tile
@@ -92,3 +94,32 @@ def test_rows_equal_across_kernels(dev, quant, down):
     s.check(short, "16-row")
     assert np.array_equal(short.view(np.uint32), tile.view(np.uint32))
     assert np.array_equal(s.run_csr(s.csr_arrays()).view(np.uint32), tile.view(np.uint32))
+
+
+def shifted(a, off, dev):
+    """A device copy of the bytes of `a` that starts `off` bytes past a 256-byte
+    boundary."""
+    t = torch.zeros(a.size + 256, dtype=torch.uint8, device=dev)[off:off + a.size]
+    t.copy_(torch.from_numpy(np.ascontiguousarray(a).view(np.uint8).reshape(-1)))
+    assert t.data_ptr() % 4 == off % 4
+    return t
+
+
+@pytest.mark.parametrize("off", [1, 2, 3])
+@pytest.mark.parametrize("quant", FORMATS, ids=lambda q: fm.NAMES[q])
+def test_q8_rows_at_any_byte(dev, quant, off):
+    """q8_K rows that do not start on a dword, which the tile's copies to LDS
+    cannot read: chunks and groups long enough for the tile, on the oracle."""
+    rows, n_tok, n = 4129, 130, 768
+    w = synth.quant_matrix(quant, rows, n, synth.rng_for(off, "shift"))
+    xq = oracle.quantize_q8_k(np.random.default_rng(off).standard_normal((n_tok, n)).astype(np.float32))
+    out = zeros_f32((n_tok, rows))
+    K.matmul_kq(out, up(w), shifted(xq, off, dev), n, rows, n_tok, row_bytes(quant, n), quant)
+    at = edge_rows(rows)
+    want, _, bound = rows_want(quant, np.ascontiguousarray(w[at]), row_bytes(quant, n), xq, n, n_tok)
+    assert_rows_close(down_np(out)[:, at], want, bound, f"{fm.NAMES[quant]} +{off}")
+    for down in (False, True):
+        s = Stage(dev, quant, down, [70, 1, 0, 129], 256, 256)
+        x = shifted(s.xq, off, dev)
+        s.check(s.run_csr(s.csr_arrays(), xq=x), "csr")
+        s.check(s.run_experts(xq=x), "experts")
