@@ -759,7 +759,7 @@ template <uint32_t Q, bool PAIR, typename G>
 __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_eu(2))) void moe_grouped_mmq_kq_kernel(
         float *__restrict__ out, const G src, const float *__restrict__ weights,
         const pulsar_block_q8_K *__restrict__ act, uint32_t k_blocks, uint32_t lim, uint32_t n_rows,
-        uint32_t n_used, uint64_t row_bytes, uint32_t act_op, uint32_t pmax, uint32_t lst_off, uint32_t bound) {
+        uint32_t n_used, uint64_t row_bytes, uint32_t act_op, uint32_t pmax, uint32_t lst_off) {
     using F = GmmqFmt<Q>;
     constexpr uint32_t NM = PAIR ? 2 : 1;
     constexpr bool kIq2 = Q == PULSAR_QUANT_IQ2_XXS;
@@ -786,9 +786,7 @@ __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_e
     }
     const uint32_t group = blockIdx.y;
     const typename G::Group grp = src.group(group);
-    // a caller's CSR whose groups are long on average is the wide tile's
-    if constexpr (std::is_same<G, CsrGroups>::value)
-        if (4ull * (src.starts[gridDim.y] - src.starts[0]) >= (uint64_t)bound * gridDim.y) return;
+    if (src.tiled()) return;  // a caller's CSR whose groups are long on average
     const pulsar_expert_ptrs &p = grp.p;
     const uint8_t *w0 = PAIR ? (const uint8_t *)p.gate : (const uint8_t *)p.down;
     const uint8_t *w1 = PAIR ? (const uint8_t *)p.up : nullptr;
@@ -1355,13 +1353,11 @@ __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_e
 // on the matrix cores; -1 for the other formats (the caller then uses the
 // lane kernels of moe.hip). `src` is the group source (CsrGroups or
 // ExpertGroups), n_group the grid's group count; lst_bytes the LDS the
-// source's pair list needs (0 for the caller's CSR). bound: a CSR whose
-// groups have bound / 4 pairs or more on average is left to the wide tile.
+// source's pair list needs (0 for the caller's CSR).
 template <typename G>
 int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, const float *weights,
                           const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
-                          uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
-                          uint32_t bound) {
+                          uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes) {
     if (quant != PULSAR_QUANT_Q2_K && quant != PULSAR_QUANT_IQ2_XXS && quant != PULSAR_QUANT_MXFP4 &&
         quant != PULSAR_QUANT_Q4_K && quant != PULSAR_QUANT_Q5_K && quant != PULSAR_QUANT_Q6_K)
         return -1;
@@ -1388,7 +1384,7 @@ int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, c
     hipLaunchKernelGGL((moe_grouped_mmq_kq_kernel<Q, P, G>),                                                     \
                        dim3((n_rows + kGqBlockRows<Q, P> - 1u) / kGqBlockRows<Q, P>, n_group),                     \
                        dim3(64u * kGqWaves<Q>), lds, pk::stream(), out, src, weights, act, k_blocks, lim, n_rows, \
-                       n_used, row_bytes, act_op, pmax, lst_off, bound)
+                       n_used, row_bytes, act_op, pmax, lst_off)
     if (quant == PULSAR_QUANT_Q2_K && pair)
         PK_GQ(PULSAR_QUANT_Q2_K, true);
     else if (quant == PULSAR_QUANT_Q2_K)
@@ -1418,9 +1414,9 @@ int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, c
 }
 template int launch_grouped_mmq_kq<CsrGroups>(bool, uint32_t, float *, const CsrGroups &, const float *,
                                               const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t, uint32_t,
-                                              uint64_t, uint32_t, uint32_t, uint32_t);
+                                              uint64_t, uint32_t, uint32_t);
 template int launch_grouped_mmq_kq<ExpertGroups>(bool, uint32_t, float *, const ExpertGroups &, const float *,
                                                  const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t, uint32_t,
-                                                 uint64_t, uint32_t, uint32_t, uint32_t);
+                                                 uint64_t, uint32_t, uint32_t);
 
 }  // namespace pk

@@ -172,6 +172,7 @@ __global__ __launch_bounds__(256) void moe_pair_grouped_kernel(
     const pulsar_expert_ptrs &p = gr.p;
     const bool nul = gr.is_null();
     if (!nul && (!p.gate || !p.up)) return;
+    if (grp.tiled()) return;
     uint32_t *lst = (uint32_t *)(acts_lds + lst_off);
     uint32_t s0, s1;
     grp.range(gr, lst, s0, s1);
@@ -256,6 +257,7 @@ __global__ __launch_bounds__(256) void moe_down_grouped_kernel(
     const pulsar_expert_ptrs &p = gr.p;
     const bool nul = gr.is_null();
     if (!nul && !p.down) return;
+    if (grp.tiled()) return;
     uint32_t *lst = (uint32_t *)(acts_lds + lst_off);
     uint32_t s0, s1;
     grp.range(gr, lst, s0, s1);
@@ -600,22 +602,21 @@ namespace pk {
 template <typename G>
 int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, const float *weights,
                           const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
-                          uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
-                          uint32_t max_pairs);
+                          uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes);
 extern template int launch_grouped_mmq_kq<CsrGroups>(bool, uint32_t, float *, const CsrGroups &, const float *,
                                                      const pulsar_block_q8_K *, uint32_t, uint32_t, uint32_t,
-                                                     uint32_t, uint64_t, uint32_t, uint32_t, uint32_t);
+                                                     uint32_t, uint64_t, uint32_t, uint32_t);
 extern template int launch_grouped_mmq_kq<ExpertGroups>(bool, uint32_t, float *, const ExpertGroups &,
                                                         const float *, const pulsar_block_q8_K *, uint32_t, uint32_t,
-                                                        uint32_t, uint32_t, uint64_t, uint32_t, uint32_t, uint32_t);
+                                                        uint32_t, uint32_t, uint64_t, uint32_t, uint32_t);
 // tile_moe.hip: the grouped stages on the wide tile
 uint32_t tile_min_quarter_pairs(bool pair, uint32_t quant);
 int launch_tile_experts(bool pair, uint32_t quant, float *out, const ExpertGroups &src, const float *weights,
                         const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
                         uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes);
 int launch_tile_csr(bool pair, uint32_t quant, float *out, const CsrGroups &src, const float *weights,
-                    const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used, uint32_t n_group,
-                    uint64_t row_bytes, uint32_t act_op, uint32_t bound);
+                    const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
+                    uint64_t row_bytes, uint32_t act_op);
 
 // The routed pairs of an ExpertGroups stage and the experts they spread over at
 // most (a caller's CSR: unknown on the host).
@@ -623,28 +624,36 @@ struct GroupSizes {
     uint32_t routed = 0, experts = 1;
 };
 
-// A grouped stage on the matrix cores; -1 where only the lane kernels have the
-// format. The routed experts' mean decides between the two kernels; a shared
-// slot's group, which holds every token, goes to the tile by its own size (top-8
-// of 256 experts and a shared one, 128 tokens: its 8 pair tiles one after the
-// other made the gate / up stage 331 us, now 138). The sizes in a caller's
-// CSR are known on the device alone: both kernels are launched, and each works
-// or ends at once by the groups' mean.
-template <typename G>
-static int grouped_mfma(bool pair, uint32_t quant, float *out, const G &grp, const float *weights,
-                        const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
-                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
-                        const GroupSizes &sizes) {
+// A grouped stage on the kernel that takes its groups: the 16-row kernel
+// (mmq.hip) or, where it has not the format or cannot hold a row, the lane
+// kernels (lane(src)), and the wide tile for long groups. The routed experts'
+// mean decides; a shared slot's group, which holds every token, goes to the tile
+// by its own size (top-8 of 256 experts and a shared one, 128 tokens: its 8 pair
+// tiles one after the other made the gate / up stage 331 us, now 138). The sizes
+// in a caller's CSR are known on the device alone: both kernels are launched,
+// and each works or ends at once by the groups' mean.
+template <typename G, typename LaneFn>
+static int grouped_stage(bool pair, uint32_t quant, float *out, G grp, const float *weights,
+                         const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
+                         uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes,
+                         const GroupSizes &sizes, LaneFn lane) {
+#ifdef PK_GRP_LANE_ONLY
+    return lane(grp);
+#endif
+    auto mmq = [&](const G &src) {
+        return launch_grouped_mmq_kq(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, n_group, row_bytes,
+                                     act_op, lst_bytes);
+    };
+    auto mmq_or_lane = [&](const G &src) {
+        const int r = mmq(src);
+        return r < 0 ? lane(src) : r;
+    };
     // rows wider than the lane kernels take are refused for every format, and
     // the tile's copies to LDS move whole dwords of act, which the other
     // kernels load at any alignment
     const bool fits = k_dim <= 16384u && (uintptr_t)act % 4u == 0u;
     const uint32_t bound = fits ? tile_min_quarter_pairs(pair, quant) : 0u;
-    auto mmq = [&](const G &src, uint32_t b) {
-        return launch_grouped_mmq_kq(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, n_group, row_bytes,
-                                     act_op, lst_bytes, b);
-    };
-    if (bound == 0u) return mmq(grp, UINT32_MAX);
+    if (bound == 0u) return mmq_or_lane(grp);
     if constexpr (std::is_same<G, ExpertGroups>::value) {
         auto tile = [&](const ExpertGroups &src, uint32_t groups) {
             return launch_tile_experts(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, groups, row_bytes,
@@ -654,59 +663,48 @@ static int grouped_mfma(bool pair, uint32_t quant, float *out, const G &grp, con
         if (grp.n_shared != 0u && grp.n_tok >= (pair ? 33u : 100u)) {
             G part = grp;
             part.which = ExpertGroups::kRouted;
-            const int r = mmq(part, UINT32_MAX);
-            if (r <= 0) return r;
+            const int r = mmq(part);
+            if (r < 0) return lane(grp);
+            if (r == 0) return r;
             part.which = ExpertGroups::kShared;
             return tile(part, grp.n_shared);
         }
-        return mmq(grp, UINT32_MAX);
+        return mmq_or_lane(grp);
     } else {
-        auto tile = [&](uint32_t b) {
-            return launch_tile_csr(pair, quant, out, grp, weights, act, k_dim, n_rows, n_used, n_group, row_bytes,
-                                   act_op, b);
-        };
-        if (n_group > 1024u) return mmq(grp, UINT32_MAX);  // more than the tile's blocks count
-        const int r = mmq(grp, bound);
-        if (r < 0) return quant == PULSAR_QUANT_Q3_K || quant == PULSAR_QUANT_IQ4_XS ? tile(0u) : r;
-        return r == 0 ? r : tile(bound);
+        if (n_group > kCsrGroups) return mmq_or_lane(grp);
+        grp.bound = bound;
+        const int r = mmq_or_lane(grp);
+        return r == 0 ? r : launch_tile_csr(pair, quant, out, grp, weights, act, k_dim, n_rows, n_used, row_bytes, act_op);
     }
 }
 
-// The grouped gate / up stage for either group source: the matrix-core
-// kernels where the format has one, else the lane kernels.
+// The grouped gate / up and down stages for either group source.
 template <typename G>
 static int pair_grouped(void *mid, const G &grp, const void *weights, const void *xq, uint32_t in_dim,
                         uint32_t mid_dim, uint32_t n_used, uint32_t n_group, uint64_t row_bytes, uint32_t quant,
                         uint32_t act_op, uint32_t lst_bytes, const GroupSizes &sizes = {}) {
-#ifndef PK_GRP_LANE_ONLY
-    {
-        const int r = grouped_mfma(true, quant, (float *)mid, grp, (const float *)weights,
-                                   (const pulsar_block_q8_K *)xq, in_dim, mid_dim, n_used, n_group, row_bytes, act_op,
-                                   lst_bytes, sizes);
-        if (r >= 0) return r;
-    }
-#endif
-    const Geo g = geo_for(quant, in_dim);
-    PairGroupedLaunch<G> f{mid, grp, weights, xq, mid_dim, n_used, n_group, act_op, row_bytes, g, lst_bytes};
-    if (!quant_ok(quant)) return reject("moe pair swiglu grouped (quant)");
-    return with_format<4>(quant, g.upl, f);
+    auto lane = [&](const G &src) {
+        const Geo g = geo_for(quant, in_dim);
+        PairGroupedLaunch<G> f{mid, src, weights, xq, mid_dim, n_used, n_group, act_op, row_bytes, g, lst_bytes};
+        if (!quant_ok(quant)) return reject("moe pair swiglu grouped (quant)");
+        return with_format<4>(quant, g.upl, f);
+    };
+    return grouped_stage(true, quant, (float *)mid, grp, (const float *)weights, (const pulsar_block_q8_K *)xq, in_dim,
+                         mid_dim, n_used, n_group, row_bytes, act_op, lst_bytes, sizes, lane);
 }
 
 template <typename G>
 static int down_grouped(void *partial, const G &grp, const void *midq, uint32_t mid_dim, uint32_t out_dim,
                         uint32_t n_used, uint32_t n_group, uint64_t row_bytes, uint32_t quant, uint32_t lst_bytes,
                         const GroupSizes &sizes = {}) {
-#ifndef PK_GRP_LANE_ONLY
-    {
-        const int r = grouped_mfma(false, quant, (float *)partial, grp, nullptr, (const pulsar_block_q8_K *)midq,
-                                   mid_dim, out_dim, n_used, n_group, row_bytes, 0u, lst_bytes, sizes);
-        if (r >= 0) return r;
-    }
-#endif
-    const Geo g = geo_for(quant, mid_dim);
-    DownGroupedLaunch<G> f{partial, grp, midq, out_dim, n_used, n_group, row_bytes, g, lst_bytes};
-    if (!quant_ok(quant)) return reject("moe down grouped (quant)");
-    return with_format<4>(quant, g.upl, f);
+    auto lane = [&](const G &src) {
+        const Geo g = geo_for(quant, mid_dim);
+        DownGroupedLaunch<G> f{partial, src, midq, out_dim, n_used, n_group, row_bytes, g, lst_bytes};
+        if (!quant_ok(quant)) return reject("moe down grouped (quant)");
+        return with_format<4>(quant, g.upl, f);
+    };
+    return grouped_stage(false, quant, (float *)partial, grp, nullptr, (const pulsar_block_q8_K *)midq, mid_dim, out_dim,
+                         n_used, n_group, row_bytes, 0u, lst_bytes, sizes, lane);
 }
 
 // ExpertGroups from the entry points' arguments (bank and shared are host
@@ -743,7 +741,8 @@ extern "C" int pulsar_moe_pair_swiglu_grouped(void *mid, const void *gptrs, cons
         n_group > 65535u || row_bytes == 0 ||
         (act_op != PULSAR_ACT_SILU && act_op != PULSAR_ACT_SWIGLU_OAI))
         return reject("moe pair swiglu grouped");
-    const CsrGroups grp{(const pulsar_expert_ptrs *)gptrs, (const uint32_t *)starts, (const uint32_t *)pairs};
+    const CsrGroups grp{(const pulsar_expert_ptrs *)gptrs, (const uint32_t *)starts, (const uint32_t *)pairs,
+                        n_group, UINT32_MAX};
     return pair_grouped(mid, grp, weights, xq, in_dim, mid_dim, n_used, n_group, row_bytes, quant, act_op, 0u);
 }
 
@@ -757,7 +756,8 @@ extern "C" int pulsar_moe_down_grouped(void *partial, const void *gptrs, const v
         out_dim == 0 || n_used == 0 || n_used > 16u || n_group == 0 || n_group > 65535u ||
         row_bytes == 0)
         return reject("moe down grouped");
-    const CsrGroups grp{(const pulsar_expert_ptrs *)gptrs, (const uint32_t *)starts, (const uint32_t *)pairs};
+    const CsrGroups grp{(const pulsar_expert_ptrs *)gptrs, (const uint32_t *)starts, (const uint32_t *)pairs,
+                        n_group, UINT32_MAX};
     return down_grouped(partial, grp, midq, mid_dim, out_dim, n_used, n_group, row_bytes, quant, 0u);
 }
 

@@ -327,10 +327,15 @@ PK_DEV SlotRoute route_slot(const float *lg, const float *rbias, uint32_t n_expe
 
 // The reference's grouped contract: a CSR by expert from the caller
 // (gptrs [n_group], starts [n_group + 1], pairs), pulsar_kernels.cu:3483-3591.
+constexpr uint32_t kCsrGroups = 1024;  // most groups whose tile counts a block of the wide tile keeps
+
 struct CsrGroups {
     const pulsar_expert_ptrs *gptrs;
     const uint32_t *starts;
     const uint32_t *pairs;
+    // Pairs per group on average, in quarters, from which the wide tile, launched
+    // after the 16-row or lane kernel, takes the stage (UINT32_MAX: no tile)
+    uint32_t n_group, bound;
 #ifdef PK_CSR_PAD
     uint8_t pad_[296];
 #endif
@@ -345,7 +350,9 @@ struct CsrGroups {
         e = starts[G.g + 1u];
     }
     PK_DEV uint32_t pair(uint32_t i, const uint32_t *) const { return pairs[i]; }
-    PK_DEV void range_block(const Group &G, uint32_t *lst, uint32_t &b, uint32_t &e) const { range(G, lst, b, e); }
+    PK_DEV bool tiled() const {
+        return bound != UINT32_MAX && 4ull * (starts[n_group] - starts[0]) >= (uint64_t)bound * n_group;
+    }
 };
 
 // One group per expert a chunk touches, in a resident bank, found from the
@@ -443,6 +450,7 @@ struct ExpertGroups {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     PK_DEV uint32_t pair(uint32_t i, const uint32_t *lst) const { return lst[i]; }
+    PK_DEV bool tiled() const { return false; }  // the host knows: it launches one kernel
     // range() by a whole block of 4 waves: each scans a quarter of the ids, all
     // its loads in flight at once, and the quarters' counts place their hits.
     // One round trip and two block barriers, where a wave that scans alone

@@ -595,6 +595,9 @@ struct Tile {
     PK_DEV static bool mine(uint32_t n, uint32_t r, uint32_t wk) { return WK == 1u || (4u * n + r) * WK / (4u * NS) == wk; }
 };
 
+// Blocks in flight at once: two per CU (256 VGPRs, 160 KiB of LDS).
+constexpr uint32_t kTileSlots = 512;
+
 // The tile of the expert groups: Tile<Q, 4, 1, NS> with the order of a token
 // slice's steps fixed. Its time goes to LDS reads that are waited for at once:
 // at 250 registers the compiler reads a step's tokens right before their MFMAs

@@ -46,9 +46,6 @@ __global__ __launch_bounds__(256, 2) void tile_gemm_kernel(float *__restrict__ o
         }
 }
 
-// Blocks in flight at once: two per CU (256 VGPRs, 160 KiB of LDS).
-constexpr uint64_t kTileSlots = 512;
-
 template <uint32_t Q, uint32_t WR, uint32_t WK, uint32_t NS>
 static uint64_t tile_items(uint32_t out_dim, uint32_t n_tok) {
     return (uint64_t)((n_tok + 16u * NS - 1u) / (16u * NS)) * ((out_dim + 32u * WR - 1u) / (32u * WR));

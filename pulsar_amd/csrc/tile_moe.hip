@@ -103,23 +103,21 @@ __global__ __launch_bounds__(256, 2) void tile_experts_kernel(float *__restrict_
                 s1 - t0 < GT::T::kTok ? s1 - t0 : GT::T::kTok, [&](uint32_t t) { return lst[t0 + t]; });
 }
 
-constexpr uint32_t kCsrGroups = 1024;  // groups whose tile counts a block keeps
-
 // A caller's CSR, whose group sizes only the device knows. A launch of at most
 // kTileSlots blocks: each counts the tiles of every group (one round trip),
 // and block b takes the (tile, row block) items b, b + grid, ...: uneven groups
-// spread evenly, and where the groups are short (fewer than bound / 4 pairs on
-// average: mmq.hip's kernel, launched before, has taken them) the blocks end
-// after one load.
+// spread evenly, and where the groups are short on average (the kernel launched
+// before has taken them) the blocks end after one load.
 template <uint32_t Q, bool PAIR, uint32_t NS>
 __global__ __launch_bounds__(256, 2) void tile_csr_kernel(float *__restrict__ out, const CsrGroups src,
                                                           const float *__restrict__ weights,
                                                           const pulsar_block_q8_K *__restrict__ act, uint32_t nb,
                                                           uint32_t n_rows, uint32_t n_used, uint64_t row_bytes,
-                                                          uint32_t act_op, uint32_t n_group, uint32_t bound) {
+                                                          uint32_t act_op) {
     using GT = GroupTile<Q, PAIR, NS>;
     constexpr uint32_t kTok = GT::T::kTok;
-    if (4ull * (src.starts[n_group] - src.starts[0]) < (uint64_t)bound * n_group) return;
+    if (!src.tiled()) return;
+    const uint32_t n_group = src.n_group;
     __shared__ __align__(16) uint8_t buf0[GT::T::kBuf];
     __shared__ __align__(16) uint8_t buf1[GT::T::kBuf];
     __shared__ uint32_t pr_l[kTok];
@@ -171,7 +169,8 @@ __global__ __launch_bounds__(256, 2) void tile_csr_kernel(float *__restrict__ ou
 }
 
 // Pairs per group, in quarters, from which the tile beats the kernel it takes
-// over from (0: no tile kernel): the 16-row kernel of mmq.hip wastes less on
+// over from (0: no tile kernel); a CSR's mean decides on the device, in either
+// kernel alike. The 16-row kernel of mmq.hip wastes less on
 // short groups and its smaller blocks keep more weight bytes in flight; for
 // Q3_K and IQ4_XS the lane kernels. Both sides by pairs per expert (us, gate /
 // up stage of 128-expert layers unless noted, the tile second): Q4_K 2048 x
@@ -221,21 +220,22 @@ int launch_tile_experts(bool pair, uint32_t quant, float *out, const ExpertGroup
     return launch_ok(pair ? "moe pair swiglu experts (tile) launch" : "moe down experts (tile) launch");
 }
 
-// The grouped stages of a caller's CSR on the tile, where the groups have bound
-// / 4 pairs or more on average (0: in any case). 128-pair tiles where the
+// The grouped stages of a caller's CSR on the tile, where src.tiled() (what the
+// kernel launched before it on the same src leaves). 128-pair tiles where the
 // format's registers allow it (Q2_K gate / up, 96 pairs per group: 685 -> 562
 // us, 16 pairs 240 / 235; Q4_K spills: 279 -> 319).
 int launch_tile_csr(bool pair, uint32_t quant, float *out, const CsrGroups &src, const float *weights,
-                    const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used, uint32_t n_group,
-                    uint64_t row_bytes, uint32_t act_op, uint32_t bound) {
+                    const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
+                    uint64_t row_bytes, uint32_t act_op) {
+    if (src.n_group > kCsrGroups) return reject("grouped tile (groups)");
 #define PK_LAUNCH(Q, P)                                                                                              \
     do {                                                                                                             \
         constexpr uint32_t NS = Q == PULSAR_QUANT_Q4_K || Q == PULSAR_QUANT_Q5_K ? 4 : 8;                            \
         const uint64_t rbs = (n_rows + GroupTile<Q, P, NS>::kRows - 1u) / GroupTile<Q, P, NS>::kRows;                \
-        const uint64_t most = rbs * n_group;                                                                         \
-        hipLaunchKernelGGL((tile_csr_kernel<Q, P, NS>), dim3((uint32_t)(most < 512u ? most : 512u)), dim3(256), 0,   \
-                           pk::stream(), out, src, weights, act, k_dim / 256u, n_rows, n_used, row_bytes, act_op,    \
-                           n_group, bound);                                                                          \
+        const uint64_t most = rbs * src.n_group;                                                                     \
+        hipLaunchKernelGGL((tile_csr_kernel<Q, P, NS>), dim3((uint32_t)(most < kTileSlots ? most : kTileSlots)),     \
+                           dim3(256), 0, pk::stream(), out, src, weights, act, k_dim / 256u, n_rows, n_used,         \
+                           row_bytes, act_op);                                                                       \
     } while (0)
     switch (quant) {
         PK_TILE_FORMATS(PK_CASE)

@@ -2,6 +2,8 @@
 the 16-row kernel (csrc/mmq.hip), the wide tile (csrc/tile_moe.hip) and the lane
 kernels (csrc/moe.hip) take a stage by the size of its groups, so every case here
 puts the same pairs on two sides of a choice or checks one side on the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -9,8 +11,8 @@ import torch
 import oracle
 from pulsar_amd import formats as fm
 from pulsar_amd import kernels as K
-from pulsar_amd import synth
-from pulsar_amd.formats import QUANT_IQ2_XXS, QUANT_Q2_K, QUANT_Q4_K, QUANT_Q5_K, QUANT_Q6_K, row_bytes
+from pulsar_amd import runtime, synth
+from pulsar_amd.formats import QUANT_IQ2_XXS, QUANT_IQ4_XS, QUANT_Q2_K, QUANT_Q3_K, QUANT_Q4_K, QUANT_Q5_K, QUANT_Q6_K, row_bytes
 from tests.gpu_util import down as down_np
 from tests.gpu_util import assert_rows_close, up, zeros_f32
 from tests.test_gpu_tile import FORMATS, SIZES, check_grouped, edge_rows, grouped_case, rows_want
@@ -123,3 +125,37 @@ def test_q8_rows_at_any_byte(dev, quant, off):
         x = shifted(s.xq, off, dev)
         s.check(s.run_csr(s.csr_arrays(), xq=x), "csr")
         s.check(s.run_experts(xq=x), "experts")
+
+
+def launches(fn):
+    """The nodes of a graph of fn's launches (recorded, not run)."""
+    hip, graph, n = runtime._hip(), ctypes.c_void_p(), ctypes.c_size_t()
+    runtime._check(hip.hipStreamBeginCapture(runtime.STREAM_PER_THREAD, runtime.CAPTURE_THREAD_LOCAL), "begin")
+    try:
+        fn()
+    finally:
+        runtime._check(hip.hipStreamEndCapture(runtime.STREAM_PER_THREAD, ctypes.byref(graph)), "end")
+    hip.hipGraphGetNodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+    runtime._check(hip.hipGraphGetNodes(graph, None, ctypes.byref(n)), "nodes")
+    hip.hipGraphDestroy(graph)
+    return n.value
+
+
+# formats and row lengths (14336 values do not fit the 16-row kernel) whose
+# short groups run on the lane kernels; sizes whose mean is on one side of the
+# tile's bound for the CSR and for the router's ids alike
+LANE_TILE = [(QUANT_Q3_K, False, 512), (QUANT_Q3_K, True, 768), (QUANT_IQ4_XS, False, 768), (QUANT_IQ4_XS, True, 512),
+             (QUANT_Q4_K, False, 14336), (QUANT_Q2_K, True, 14336), (QUANT_Q6_K, True, 14336)]
+
+
+@pytest.mark.parametrize("long", [False, True])
+@pytest.mark.parametrize("quant,down,cols", LANE_TILE, ids=lambda v: str(v))
+def test_lane_or_tile_by_the_mean(dev, quant, down, cols, long):
+    """A CSR of short groups runs on the lane kernels, of long ones on the tile,
+    as the router's ids do: both on the oracle, and equal bit for bit."""
+    sizes = [40, 33, 50] if long else [1] * 40
+    s = Stage(dev, quant, down, sizes, *((70, cols) if down else (cols, 70)), n_used=1)
+    csr, ids = s.run_csr(s.csr_arrays()), s.run_experts()
+    s.check(csr, "csr")
+    s.check(ids, "experts")
+    assert np.array_equal(csr.view(np.uint32), ids.view(np.uint32))
