@@ -147,6 +147,23 @@ int pulsar_moe_down_grouped(void *partial, const void *gptrs, const void *starts
                             uint32_t out_dim, uint32_t n_used, uint32_t n_group,
                             uint64_t row_bytes, uint32_t quant);
 
+/* The two grouped calls for a caller that knows how many pairs its CSR lists
+ * at most (the capacity of `pairs`; starts[n_group] - starts[0] <= max_pairs).
+ * The calls above do not: where the tile may take the stage they launch two
+ * kernels, each of which works or ends at once by the groups' mean on the
+ * device. These leave the second out where max_pairs / n_group shows the
+ * groups short. The same rows. */
+int pulsar_moe_pair_swiglu_grouped_bounded(void *mid, const void *gptrs, const void *starts,
+                                           const void *pairs, const void *weights,
+                                           const void *xq, uint32_t in_dim, uint32_t mid_dim,
+                                           uint32_t n_used, uint32_t n_group,
+                                           uint64_t row_bytes, uint32_t quant,
+                                           uint32_t act_op, uint32_t max_pairs);
+int pulsar_moe_down_grouped_bounded(void *partial, const void *gptrs, const void *starts,
+                                    const void *pairs, const void *midq, uint32_t mid_dim,
+                                    uint32_t out_dim, uint32_t n_used, uint32_t n_group,
+                                    uint64_t row_bytes, uint32_t quant, uint32_t max_pairs);
+
 /* out[t][r] = sum_s partial[t][s][r] in slot order. Replaces
  * pulsar_moe_slot_sum (pulsar_kernels.cu:3651). */
 int pulsar_moe_slot_sum(void *out, const void *partial, uint32_t out_dim,

@@ -26,6 +26,9 @@ SIGNATURES = {
     "pulsar_moe_down": [_vp, _vp, _vp, _u32, _u32, _u32, _u32, _u64, _u32],
     "pulsar_moe_pair_swiglu_grouped": [_vp, _vp, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32, _u64, _u32, _u32],
     "pulsar_moe_down_grouped": [_vp, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32, _u64, _u32],
+    "pulsar_moe_pair_swiglu_grouped_bounded": [_vp, _vp, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32, _u64, _u32,
+                                               _u32, _u32],
+    "pulsar_moe_down_grouped_bounded": [_vp, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32, _u64, _u32, _u32],
     "pulsar_moe_slot_sum": [_vp, _vp, _u32, _u32, _u32],
     "pulsar_moe_down_bias": [_vp, _vp, _vp, _u32, _u32, _u32],
     "pulsar_router_select": [_vp, _vp, _vp, _vp, _u32, _u32, _f32, _u32, _u32, _u32],

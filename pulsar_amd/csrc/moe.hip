@@ -618,10 +618,11 @@ int launch_tile_csr(bool pair, uint32_t quant, float *out, const CsrGroups &src,
                     const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
                     uint64_t row_bytes, uint32_t act_op);
 
-// The routed pairs of an ExpertGroups stage and the experts they spread over at
-// most (a caller's CSR: unknown on the host).
+// What the host knows of the groups' sizes. ExpertGroups: the routed pairs and
+// the experts they spread over at most; a caller's CSR: the most pairs it can
+// list.
 struct GroupSizes {
-    uint32_t routed = 0, experts = 1;
+    uint32_t pairs, experts = 1;
 };
 
 // A grouped stage on the kernel that takes its groups: the 16-row kernel
@@ -631,7 +632,10 @@ struct GroupSizes {
 // by its own size (top-8 of 256 experts and a shared one, 128 tokens: its 8 pair
 // tiles one after the other made the gate / up stage 331 us, now 138). The sizes
 // in a caller's CSR are known on the device alone: both kernels are launched,
-// and each works or ends at once by the groups' mean.
+// and each works or ends at once by the groups' mean, unless the most pairs it
+// can list make short groups of them (a launch that ends at once takes 1.3-1.6
+// us: Q2_K, 128 pairs in 128 groups, gate / up 76.7 us alone and 78.0 with it,
+// down 42.2 and 43.8).
 template <typename G, typename LaneFn>
 static int grouped_stage(bool pair, uint32_t quant, float *out, G grp, const float *weights,
                          const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
@@ -659,7 +663,7 @@ static int grouped_stage(bool pair, uint32_t quant, float *out, G grp, const flo
             return launch_tile_experts(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, groups, row_bytes,
                                        act_op, lst_bytes);
         };
-        if (4u * sizes.routed >= bound * sizes.experts) return tile(grp, n_group);
+        if (4u * sizes.pairs >= bound * sizes.experts) return tile(grp, n_group);
         if (grp.n_shared != 0u && grp.n_tok >= (pair ? 33u : 100u)) {
             G part = grp;
             part.which = ExpertGroups::kRouted;
@@ -671,7 +675,7 @@ static int grouped_stage(bool pair, uint32_t quant, float *out, G grp, const flo
         }
         return mmq_or_lane(grp);
     } else {
-        if (n_group > kCsrGroups) return mmq_or_lane(grp);
+        if (n_group > kCsrGroups || 4ull * sizes.pairs < (uint64_t)bound * n_group) return mmq_or_lane(grp);
         grp.bound = bound;
         const int r = mmq_or_lane(grp);
         return r == 0 ? r : launch_tile_csr(pair, quant, out, grp, weights, act, k_dim, n_rows, n_used, row_bytes, act_op);
@@ -682,7 +686,7 @@ static int grouped_stage(bool pair, uint32_t quant, float *out, G grp, const flo
 template <typename G>
 static int pair_grouped(void *mid, const G &grp, const void *weights, const void *xq, uint32_t in_dim,
                         uint32_t mid_dim, uint32_t n_used, uint32_t n_group, uint64_t row_bytes, uint32_t quant,
-                        uint32_t act_op, uint32_t lst_bytes, const GroupSizes &sizes = {}) {
+                        uint32_t act_op, uint32_t lst_bytes, const GroupSizes &sizes) {
     auto lane = [&](const G &src) {
         const Geo g = geo_for(quant, in_dim);
         PairGroupedLaunch<G> f{mid, src, weights, xq, mid_dim, n_used, n_group, act_op, row_bytes, g, lst_bytes};
@@ -696,7 +700,7 @@ static int pair_grouped(void *mid, const G &grp, const void *weights, const void
 template <typename G>
 static int down_grouped(void *partial, const G &grp, const void *midq, uint32_t mid_dim, uint32_t out_dim,
                         uint32_t n_used, uint32_t n_group, uint64_t row_bytes, uint32_t quant, uint32_t lst_bytes,
-                        const GroupSizes &sizes = {}) {
+                        const GroupSizes &sizes) {
     auto lane = [&](const G &src) {
         const Geo g = geo_for(quant, mid_dim);
         DownGroupedLaunch<G> f{partial, src, midq, out_dim, n_used, n_group, row_bytes, g, lst_bytes};
@@ -725,12 +729,12 @@ static ExpertGroups expert_groups(const void *selected, const void *active, cons
 }
 }  // namespace pk
 
-extern "C" int pulsar_moe_pair_swiglu_grouped(void *mid, const void *gptrs, const void *starts,
-                                              const void *pairs, const void *weights,
-                                              const void *xq, uint32_t in_dim, uint32_t mid_dim,
-                                              uint32_t n_used, uint32_t n_group,
-                                              uint64_t row_bytes, uint32_t quant,
-                                              uint32_t act_op) {
+extern "C" int pulsar_moe_pair_swiglu_grouped_bounded(void *mid, const void *gptrs, const void *starts,
+                                                      const void *pairs, const void *weights,
+                                                      const void *xq, uint32_t in_dim, uint32_t mid_dim,
+                                                      uint32_t n_used, uint32_t n_group,
+                                                      uint64_t row_bytes, uint32_t quant,
+                                                      uint32_t act_op, uint32_t max_pairs) {
     quant &= ~PULSAR_QUANT_A4_OK;
     // MXFP4 rows need only whole 32-value blocks (a superset of the
     // reference's in_dim % 256 contract, which keeps gpt-oss's 2880 off the
@@ -743,13 +747,24 @@ extern "C" int pulsar_moe_pair_swiglu_grouped(void *mid, const void *gptrs, cons
         return reject("moe pair swiglu grouped");
     const CsrGroups grp{(const pulsar_expert_ptrs *)gptrs, (const uint32_t *)starts, (const uint32_t *)pairs,
                         n_group, UINT32_MAX};
-    return pair_grouped(mid, grp, weights, xq, in_dim, mid_dim, n_used, n_group, row_bytes, quant, act_op, 0u);
+    return pair_grouped(mid, grp, weights, xq, in_dim, mid_dim, n_used, n_group, row_bytes, quant, act_op, 0u,
+                        GroupSizes{max_pairs});
 }
 
-extern "C" int pulsar_moe_down_grouped(void *partial, const void *gptrs, const void *starts,
-                                       const void *pairs, const void *midq, uint32_t mid_dim,
-                                       uint32_t out_dim, uint32_t n_used, uint32_t n_group,
-                                       uint64_t row_bytes, uint32_t quant) {
+extern "C" int pulsar_moe_pair_swiglu_grouped(void *mid, const void *gptrs, const void *starts,
+                                              const void *pairs, const void *weights,
+                                              const void *xq, uint32_t in_dim, uint32_t mid_dim,
+                                              uint32_t n_used, uint32_t n_group,
+                                              uint64_t row_bytes, uint32_t quant,
+                                              uint32_t act_op) {
+    return pulsar_moe_pair_swiglu_grouped_bounded(mid, gptrs, starts, pairs, weights, xq, in_dim, mid_dim, n_used,
+                                                  n_group, row_bytes, quant, act_op, UINT32_MAX);
+}
+
+extern "C" int pulsar_moe_down_grouped_bounded(void *partial, const void *gptrs, const void *starts,
+                                               const void *pairs, const void *midq, uint32_t mid_dim,
+                                               uint32_t out_dim, uint32_t n_used, uint32_t n_group,
+                                               uint64_t row_bytes, uint32_t quant, uint32_t max_pairs) {
     quant &= ~PULSAR_QUANT_A4_OK;
     const uint32_t k_mult = quant == PULSAR_QUANT_MXFP4 ? 32u : 256u;
     if (!partial || !gptrs || !starts || !pairs || !midq || mid_dim == 0 || mid_dim % k_mult != 0 ||
@@ -758,7 +773,16 @@ extern "C" int pulsar_moe_down_grouped(void *partial, const void *gptrs, const v
         return reject("moe down grouped");
     const CsrGroups grp{(const pulsar_expert_ptrs *)gptrs, (const uint32_t *)starts, (const uint32_t *)pairs,
                         n_group, UINT32_MAX};
-    return down_grouped(partial, grp, midq, mid_dim, out_dim, n_used, n_group, row_bytes, quant, 0u);
+    return down_grouped(partial, grp, midq, mid_dim, out_dim, n_used, n_group, row_bytes, quant, 0u,
+                        GroupSizes{max_pairs});
+}
+
+extern "C" int pulsar_moe_down_grouped(void *partial, const void *gptrs, const void *starts,
+                                       const void *pairs, const void *midq, uint32_t mid_dim,
+                                       uint32_t out_dim, uint32_t n_used, uint32_t n_group,
+                                       uint64_t row_bytes, uint32_t quant) {
+    return pulsar_moe_down_grouped_bounded(partial, gptrs, starts, pairs, midq, mid_dim, out_dim, n_used, n_group,
+                                           row_bytes, quant, UINT32_MAX);
 }
 
 // Shared checks of the expert-indexed grouped entry points.

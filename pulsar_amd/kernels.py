@@ -73,12 +73,19 @@ def moe_down(out, ptrs, mid, mid_dim: int, out_dim: int, n_used: int, n_tok: int
     )
 
 
+def _capacity(pairs) -> int:
+    """The most pairs a CSR over `pairs` can list (a raw address: unknown)."""
+    if not hasattr(pairs, "data_ptr"):
+        return 0xFFFFFFFF
+    return min(pairs.numel() * pairs.element_size() // 4, 0xFFFFFFFF)
+
+
 def moe_pair_swiglu_grouped(mid, gptrs, starts, pairs, weights, xq, in_dim: int, mid_dim: int,
                             n_used: int, n_group: int, row_bytes: int, quant: int, act_op: int) -> None:
     _check(
-        _lib.load().pulsar_moe_pair_swiglu_grouped(_ptr(mid), _ptr(gptrs), _ptr(starts), _ptr(pairs),
-                                                   _ptr(weights), _ptr(xq), in_dim, mid_dim, n_used,
-                                                   n_group, row_bytes, quant, act_op),
+        _lib.load().pulsar_moe_pair_swiglu_grouped_bounded(_ptr(mid), _ptr(gptrs), _ptr(starts), _ptr(pairs),
+                                                           _ptr(weights), _ptr(xq), in_dim, mid_dim, n_used,
+                                                           n_group, row_bytes, quant, act_op, _capacity(pairs)),
         "moe_pair_swiglu_grouped",
     )
 
@@ -86,9 +93,9 @@ def moe_pair_swiglu_grouped(mid, gptrs, starts, pairs, weights, xq, in_dim: int,
 def moe_down_grouped(partial, gptrs, starts, pairs, midq, mid_dim: int, out_dim: int, n_used: int,
                      n_group: int, row_bytes: int, quant: int) -> None:
     _check(
-        _lib.load().pulsar_moe_down_grouped(_ptr(partial), _ptr(gptrs), _ptr(starts), _ptr(pairs),
-                                            _ptr(midq), mid_dim, out_dim, n_used, n_group, row_bytes,
-                                            quant),
+        _lib.load().pulsar_moe_down_grouped_bounded(_ptr(partial), _ptr(gptrs), _ptr(starts), _ptr(pairs),
+                                                    _ptr(midq), mid_dim, out_dim, n_used, n_group, row_bytes,
+                                                    quant, _capacity(pairs)),
         "moe_down_grouped",
     )
 

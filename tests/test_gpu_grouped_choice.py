@@ -159,3 +159,34 @@ def test_lane_or_tile_by_the_mean(dev, quant, down, cols, long):
     s.check(csr, "csr")
     s.check(ids, "experts")
     assert np.array_equal(csr.view(np.uint32), ids.view(np.uint32))
+
+
+@pytest.mark.parametrize("down", [False, True])
+@pytest.mark.parametrize("quant", FORMATS, ids=lambda q: fm.NAMES[q])
+def test_short_csr_is_one_launch(dev, quant, down):
+    """A CSR that cannot list enough pairs for the tile (here 40 in 60 groups)
+    takes one launch; with the capacity unknown, as through a raw address, or
+    with room for long groups it takes two, and the rows are the same."""
+    s = Stage(dev, quant, down, [1] * 40, *((70, 512) if down else (512, 70)))
+    g, starts, pairs = (up(a) for a in s.csr_arrays(pad=20))
+    roomy = torch.zeros(4 * 4096, dtype=torch.uint8, device=dev)
+    roomy[:pairs.numel()] = pairs
+
+    def stage(pairs):
+        out = torch.zeros((s.T * s.n_used, s.rows), dtype=torch.float32, device=dev)
+        torch.cuda.synchronize()
+
+        def call():
+            if down:
+                K.moe_down_grouped(out, g, starts, pairs, s.d_xq, s.cols, s.rows, s.n_used, 60, s.rb, quant)
+            else:
+                K.moe_pair_swiglu_grouped(out, g, starts, pairs, s.d_w, s.d_xq, s.cols, s.rows, s.n_used, 60, s.rb,
+                                          quant, 0)
+        n = launches(call)
+        call()
+        return n, down_np(out).view(np.uint32)
+
+    (n1, a), (n2, b), (n3, c) = stage(pairs), stage(pairs.data_ptr()), stage(roomy)
+    assert (n1, n2, n3) == (1, 2, 2)
+    assert np.array_equal(a, b) and np.array_equal(a, c)
+    s.check(a.view(np.float32), "csr")
