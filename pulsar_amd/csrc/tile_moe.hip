@@ -103,8 +103,8 @@ __global__ __launch_bounds__(256, 2) void tile_experts_kernel(float *__restrict_
                 s1 - t0 < GT::T::kTok ? s1 - t0 : GT::T::kTok, [&](uint32_t t) { return lst[t0 + t]; });
 }
 
-// A caller's CSR, whose group sizes only the device knows. A launch of at most
-// kTileSlots blocks: each counts the tiles of every group (one round trip),
+// A caller's CSR, whose group sizes only the device knows. A launch of
+// kTileSlots blocks, however few the groups: each counts the tiles of every group (one round trip),
 // and block b takes the (tile, row block) items b, b + grid, ...: uneven groups
 // spread evenly, and where the groups are short on average (the kernel launched
 // before has taken them) the blocks end after one load.
@@ -231,11 +231,8 @@ int launch_tile_csr(bool pair, uint32_t quant, float *out, const CsrGroups &src,
 #define PK_LAUNCH(Q, P)                                                                                              \
     do {                                                                                                             \
         constexpr uint32_t NS = Q == PULSAR_QUANT_Q4_K || Q == PULSAR_QUANT_Q5_K ? 4 : 8;                            \
-        const uint64_t rbs = (n_rows + GroupTile<Q, P, NS>::kRows - 1u) / GroupTile<Q, P, NS>::kRows;                \
-        const uint64_t most = rbs * src.n_group;                                                                     \
-        hipLaunchKernelGGL((tile_csr_kernel<Q, P, NS>), dim3((uint32_t)(most < kTileSlots ? most : kTileSlots)),     \
-                           dim3(256), 0, pk::stream(), out, src, weights, act, k_dim / 256u, n_rows, n_used,         \
-                           row_bytes, act_op);                                                                       \
+        hipLaunchKernelGGL((tile_csr_kernel<Q, P, NS>), dim3(kTileSlots), dim3(256), 0, pk::stream(), out, src,      \
+                           weights, act, k_dim / 256u, n_rows, n_used, row_bytes, act_op);                           \
     } while (0)
     switch (quant) {
         PK_TILE_FORMATS(PK_CASE)

@@ -52,16 +52,22 @@ class Stage:
         starts = (skip + np.concatenate([[0], np.cumsum([len(v) for v in lists])])).astype(np.uint32)
         return g, starts, pairs
 
-    def run_csr(self, arrays, out=None, xq=None):
-        g, starts, pairs = (up(a) for a in arrays)
-        n_group = len(arrays[1]) - 1
-        out = torch.zeros((self.T * self.n_used, self.rows), dtype=torch.float32, device=self.dev) if out is None else out
+    def queue_csr(self, dev_arrays, n_group, out, xq=None):
+        g, starts, pairs = dev_arrays
         xq = self.d_xq if xq is None else xq
         if self.down:
             K.moe_down_grouped(out, g, starts, pairs, xq, self.cols, self.rows, self.n_used, n_group, self.rb, self.quant)
         else:
             K.moe_pair_swiglu_grouped(out, g, starts, pairs, self.d_w, xq, self.cols, self.rows, self.n_used, n_group,
                                       self.rb, self.quant, 0)
+
+    def zeros(self):
+        return torch.zeros((self.T * self.n_used, self.rows), dtype=torch.float32, device=self.dev)
+
+    def run_csr(self, arrays, xq=None):
+        out, dev_arrays = self.zeros(), [up(a) for a in arrays]
+        torch.cuda.synchronize()
+        self.queue_csr(dev_arrays, len(arrays[1]) - 1, out, xq)
         return down_np(out)
 
     def run_experts(self, xq=None):
@@ -127,8 +133,13 @@ def test_q8_rows_at_any_byte(dev, quant, off):
         s.check(s.run_experts(xq=x), "experts")
 
 
+class KernelNode(ctypes.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                ("grid", ctypes.c_uint * 3), ("args", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
 def launches(fn):
-    """The nodes of a graph of fn's launches (recorded, not run)."""
+    """The kernel nodes of a graph of fn's launches (recorded, not run)."""
     hip, graph, n = runtime._hip(), ctypes.c_void_p(), ctypes.c_size_t()
     runtime._check(hip.hipStreamBeginCapture(runtime.STREAM_PER_THREAD, runtime.CAPTURE_THREAD_LOCAL), "begin")
     try:
@@ -136,9 +147,17 @@ def launches(fn):
     finally:
         runtime._check(hip.hipStreamEndCapture(runtime.STREAM_PER_THREAD, ctypes.byref(graph)), "end")
     hip.hipGraphGetNodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+    hip.hipGraphKernelNodeGetParams.argtypes = [ctypes.c_void_p, ctypes.POINTER(KernelNode)]
     runtime._check(hip.hipGraphGetNodes(graph, None, ctypes.byref(n)), "nodes")
+    nodes = (ctypes.c_void_p * n.value)()
+    runtime._check(hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)), "nodes")
+    out = []
+    for node in nodes:
+        k = KernelNode()
+        runtime._check(hip.hipGraphKernelNodeGetParams(node, ctypes.byref(k)), "node")
+        out.append(k)
     hip.hipGraphDestroy(graph)
-    return n.value
+    return out
 
 
 # formats and row lengths (14336 values do not fit the 16-row kernel) whose
@@ -173,16 +192,13 @@ def test_short_csr_is_one_launch(dev, quant, down):
     roomy[:pairs.numel()] = pairs
 
     def stage(pairs):
-        out = torch.zeros((s.T * s.n_used, s.rows), dtype=torch.float32, device=dev)
+        out = s.zeros()
         torch.cuda.synchronize()
 
         def call():
-            if down:
-                K.moe_down_grouped(out, g, starts, pairs, s.d_xq, s.cols, s.rows, s.n_used, 60, s.rb, quant)
-            else:
-                K.moe_pair_swiglu_grouped(out, g, starts, pairs, s.d_w, s.d_xq, s.cols, s.rows, s.n_used, 60, s.rb,
-                                          quant, 0)
-        n = launches(call)
+            s.queue_csr((g, starts, pairs), 60, out)
+
+        n = len(launches(call))
         call()
         return n, down_np(out).view(np.uint32)
 
@@ -190,3 +206,15 @@ def test_short_csr_is_one_launch(dev, quant, down):
     assert (n1, n2, n3) == (1, 2, 2)
     assert np.array_equal(a, b) and np.array_equal(a, c)
     s.check(a.view(np.float32), "csr")
+
+
+@pytest.mark.parametrize("down", [False, True])
+def test_few_long_groups_fill_the_chip(dev, down):
+    """One group of many pair tiles is spread over as many blocks as many
+    groups are: the tiles count, not the groups."""
+    s = Stage(dev, QUANT_Q4_K, down, [1500], *((330, 512) if down else (512, 330)))
+    dev_arrays = [up(a) for a in s.csr_arrays()]
+    out = s.zeros()
+    torch.cuda.synchronize()
+    assert launches(lambda: s.queue_csr(dev_arrays, 1, out))[-1].grid[0] == 512
+    s.check(s.run_csr(s.csr_arrays()), "csr")
