@@ -1349,21 +1349,14 @@ __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_e
     }
 }
 
-// Grouped MoE stages of Q2_K, IQ2_XXS, MXFP4, Q4_K, Q5_K and Q6_K experts
-// on the matrix cores; -1 for the other formats (the caller then uses the
-// lane kernels of moe.hip). `src` is the group source (CsrGroups or
-// ExpertGroups), n_group the grid's group count; lst_bytes the LDS the
-// source's pair list needs (0 for the caller's CSR).
-template <typename G>
-int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, const float *weights,
-                          const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
-                          uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes) {
+// Pairs of an expert in one tile of a stage (each tile is a pass over the
+// expert's weights); 0 where the kernel has not the format or cannot hold one
+// pair's row.
+uint32_t grouped_mmq_pairs(bool pair, uint32_t quant, uint32_t k_dim, uint32_t lst_bytes) {
     if (quant != PULSAR_QUANT_Q2_K && quant != PULSAR_QUANT_IQ2_XXS && quant != PULSAR_QUANT_MXFP4 &&
         quant != PULSAR_QUANT_Q4_K && quant != PULSAR_QUANT_Q5_K && quant != PULSAR_QUANT_Q6_K)
-        return -1;
-    const uint32_t k_blocks = (k_dim + 255u) / 256u;
-    const uint32_t lim = quant == PULSAR_QUANT_MXFP4 ? k_dim / 32u : k_blocks;
-    const uint32_t per_pair = act_row_pitch(k_blocks);
+        return 0u;
+    const uint32_t per_pair = act_row_pitch((k_dim + 255u) / 256u);
     // MXFP4 layers route many pairs to each expert (gpt-oss: 64 tokens x 4 of
     // 32 experts), so their tiles take more pairs per weight pass
     // Gate / up tiles of 4096-value rows hold 5 pairs instead of 3 (4880 bytes
@@ -1375,9 +1368,24 @@ int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, c
     const uint32_t budget = quant == PULSAR_QUANT_MXFP4          ? kGqActLdsMx
                             : pair && lst_bytes <= 1024u ? kGqActLdsPair
                                                          : kGqActLds;
-    if (per_pair > budget) return -1;  // one pair's row does not fit: lane kernels
-    uint32_t pmax = budget / per_pair;
-    pmax = pmax < kGqPairs ? pmax : kGqPairs;
+    const uint32_t pmax = budget / per_pair;
+    return pmax < kGqPairs ? pmax : kGqPairs;
+}
+
+// Grouped MoE stages of Q2_K, IQ2_XXS, MXFP4, Q4_K, Q5_K and Q6_K experts
+// on the matrix cores; -1 where grouped_mmq_pairs is 0 (the caller then uses
+// the lane kernels of moe.hip). `src` is the group source (CsrGroups or
+// ExpertGroups), n_group the grid's group count; lst_bytes the LDS the
+// source's pair list needs (0 for the caller's CSR).
+template <typename G>
+int launch_grouped_mmq_kq(bool pair, uint32_t quant, float *out, const G &src, const float *weights,
+                          const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
+                          uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes) {
+    const uint32_t pmax = grouped_mmq_pairs(pair, quant, k_dim, lst_bytes);
+    if (pmax == 0u) return -1;
+    const uint32_t k_blocks = (k_dim + 255u) / 256u;
+    const uint32_t lim = quant == PULSAR_QUANT_MXFP4 ? k_dim / 32u : k_blocks;
+    const uint32_t per_pair = act_row_pitch(k_blocks);
     const uint32_t lst_off = (pmax * per_pair + 15u) & ~15u;
     const size_t lds = (size_t)lst_off + lst_bytes;
 #define PK_GQ(Q, P)                                                                                              \

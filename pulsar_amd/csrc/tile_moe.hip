@@ -170,27 +170,53 @@ __global__ __launch_bounds__(256, 2) void tile_csr_kernel(float *__restrict__ ou
 
 // Pairs per group, in quarters, from which the tile beats the kernel it takes
 // over from (0: no tile kernel); a CSR's mean decides on the device, in either
-// kernel alike. The 16-row kernel of mmq.hip wastes less on
-// short groups and its smaller blocks keep more weight bytes in flight; for
-// Q3_K and IQ4_XS the lane kernels. Both sides by pairs per expert (us, gate /
-// up stage of 128-expert layers unless noted, the tile second): Q4_K 2048 x
-// 768: 4: 66 / 66, 6: 87 / 69, 14: 152 / 73; Q2_K 4096 x 1536: 2.5: 145 / 190,
-// 4: 210 / 195, 14: 577 / 207; IQ2_XXS: 4: 255 / 345, 6: 365 / 347, 14: 693 / 353;
-// Q5_K: 6: 107 / 96, 14: 198 / 106; IQ4_XS: 1: 62 / 68, 2.5: 124 / 83, 14: 515 /
-// 93; Q3_K 64 experts of 2048 x 1024: 0.8: 35 / 44, 1.5: 57 / 51, 21: 568 / 62.
-// Down stages, whose rows have few super-blocks: Q6_K 768 x 2048: 16: 98 / 115;
-// Q2_K 1536 x 4096: 14: 186 / 124; IQ2_XXS: 14: 191 / 195; Q5_K: 14: 77 / 58.
-uint32_t tile_min_quarter_pairs(bool pair, uint32_t quant) {
+// kernel alike. nb: super-blocks of a row; groups, n_rows: the stage's;
+// pmax: pairs per tile of the 16-row kernel (mmq.hip), 0 where it cannot hold a
+// row.
+//
+// The 16-row kernel reads an expert's weights once per pmax pairs, the tile once
+// per 64 with more work per super-block: a group of m pairs costs the one about
+// m / pmax + 1/2 passes and the other a fixed number of them, which grows with
+// the row length (a pass over a short row is mostly its staging) up to a bound.
+// That number, from 1400 stages of 10 layer shapes timed on both (8 to 256
+// experts, 2 to 56 super-blocks, 1 to 256 pairs per expert, weights from HBM),
+// in hundredths: none of them is more than 1% slower than on the 16-row kernel,
+// and the faster kernel is missed by 0.7% on average. Some of them:
+// gate / up, us by pairs per expert, 16-row / tile: IQ2_XXS 128 experts of 1536
+// x 4096, 4: 239 / 321, 6: 331 / 330, 12: 615 / 338; 32 of 2816 x 2816, 6: 82 /
+// 123, 10: 139 / 126; Q2_K 16 of 6400 x 4096, 4: 77 / 90, 8: 133 / 117; Q5_K 32
+// of 2816 x 2816, 5: 94 / 120, 8: 133 / 123; Q4_K 128 of 768 x 2048, 4: 74 / 70;
+// down, Q6_K 128 of 2048 x 768, 12: 88 / 97, 16: 112 / 100.
+// Where a launch's blocks leave CUs idle the 16-row kernel's passes are one
+// after the other (8 experts of 2048 x 4096, IQ2_XXS, 4: 56 / 48).
+// Against the lane kernels the line lies at 2 to 3 pairs for the rows the
+// 16-row kernel cannot hold (8 experts of 4096 x 14336, down, lane / tile, 2:
+// Q6_K 216 / 188, Q4_K 169 / 103, IQ2_XXS 119 / 163; 3: IQ2_XXS 179 / 164) and
+// at 1.5 for Q3_K and IQ4_XS (IQ4_XS 128 of 768 x 2048, 1: 51 / 57, 1.5: 89 /
+// 72), whose down stages of one or two super-blocks reach it at 2.
+uint32_t tile_min_quarter_pairs(bool pair, uint32_t quant, uint32_t nb, uint32_t n_rows, uint32_t groups,
+                                uint32_t pmax) {
+    struct Passes {
+        uint32_t base, per_sb, most;
+    } p;
     switch (quant) {
-    case PULSAR_QUANT_Q4_K:
-    case PULSAR_QUANT_Q5_K: return pair ? 20u : 48u;
-    case PULSAR_QUANT_Q6_K: return pair ? 48u : 128u;
-    case PULSAR_QUANT_Q2_K: return pair ? 16u : 48u;
-    case PULSAR_QUANT_IQ2_XXS: return pair ? 24u : 60u;
+    case PULSAR_QUANT_Q4_K: p = pair ? Passes{70, 5, 150} : Passes{45, 10, 160}; break;
+    case PULSAR_QUANT_Q5_K: p = pair ? Passes{93, 5, 180} : Passes{68, 13, 170}; break;
+    case PULSAR_QUANT_Q6_K: p = pair ? Passes{100, 8, 220} : Passes{90, 15, 290}; break;
+    case PULSAR_QUANT_Q2_K: p = pair ? Passes{84, 6, 180} : Passes{65, 13, 170}; break;
+    case PULSAR_QUANT_IQ2_XXS: p = pair ? Passes{90, 10, 260} : Passes{120, 15, 240}; break;
     case PULSAR_QUANT_Q3_K:
-    case PULSAR_QUANT_IQ4_XS: return 6u;
+    case PULSAR_QUANT_IQ4_XS: return !pair && nb <= 2u ? 8u : 6u;
     default: return 0u;
     }
+    if (pmax == 0u) return quant == PULSAR_QUANT_IQ2_XXS ? 12u : 8u;
+    uint32_t passes = p.base + p.per_sb * nb;
+    if (passes > p.most) passes = p.most;
+    const uint32_t rows = pair ? 64u : 128u;
+    if (quant != PULSAR_QUANT_Q6_K && (uint64_t)((n_rows + rows - 1u) / rows) * groups <= 256u && passes > 130u)
+        passes = 130u;
+    const uint32_t bound = passes > 50u ? ((passes - 50u) * pmax * 4u + 99u) / 100u : 0u;
+    return bound > 8u ? bound : 8u;
 }
 
 #define PK_TILE_FORMATS(F)                                                                                            \

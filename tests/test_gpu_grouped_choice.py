@@ -218,3 +218,35 @@ def test_few_long_groups_fill_the_chip(dev, down):
     torch.cuda.synchronize()
     assert launches(lambda: s.queue_csr(dev_arrays, 1, out))[-1].grid[0] == 512
     s.check(s.run_csr(s.csr_arrays()), "csr")
+
+
+# (format, down, experts, rows, cols, tokens, top): stages of which the 16-row
+# kernel was timed faster than the tile (at the left of the line between the
+# two, by format, row length and pairs per expert), and slower
+ON_ROW16 = [(QUANT_IQ2_XXS, False, 32, 2816, 2816, 48, 4), (QUANT_IQ2_XXS, False, 8, 14336, 4096, 24, 2),
+            (QUANT_Q2_K, False, 16, 6400, 4096, 40, 2), (QUANT_Q2_K, False, 32, 2816, 2816, 32, 4),
+            (QUANT_Q5_K, False, 32, 2816, 2816, 40, 4), (QUANT_IQ2_XXS, False, 128, 768, 2048, 96, 8),
+            (QUANT_IQ2_XXS, True, 128, 2048, 768, 256, 8), (QUANT_Q6_K, True, 128, 2048, 768, 192, 8)]
+ON_TILE = [(QUANT_IQ2_XXS, False, 32, 2816, 2816, 80, 4), (QUANT_Q2_K, False, 128, 1536, 4096, 80, 8),
+           (QUANT_Q4_K, False, 128, 768, 2048, 96, 8), (QUANT_Q5_K, False, 32, 2816, 2816, 80, 4),
+           (QUANT_Q6_K, True, 128, 2048, 768, 256, 8), (QUANT_Q6_K, True, 8, 4096, 14336, 24, 2)]
+
+
+@pytest.mark.parametrize("stage", ON_ROW16 + ON_TILE, ids=lambda s: "-".join(map(str, s)))
+def test_choice_by_measured_crossover(dev, stage):
+    """The kernel a stage of the router's ids is recorded on (nothing runs):
+    the tile's only dynamic LDS is the pair list, 4 bytes a routed pair."""
+    quant, down, E, rows, cols, T, k = stage
+    bank = K.ExpertBank(256, 256, 256, None, None, None, 0, 0, 0, 0, 0, 0)  # addresses are not read
+    buf = torch.zeros(256, dtype=torch.uint8, device=dev)
+
+    def call():
+        if down:
+            K.moe_down_experts(buf, buf, buf, buf, bank, E, [], T, k, cols, rows, row_bytes(quant, cols), quant)
+        else:
+            K.moe_pair_swiglu_experts(buf, buf, buf, buf, buf, bank, E, [], T, k, cols, rows, row_bytes(quant, cols),
+                                      quant, 0)
+
+    nodes = launches(call)
+    assert len(nodes) == 1
+    assert (nodes[0].shared == 4 * T * k) == (stage in ON_TILE)
