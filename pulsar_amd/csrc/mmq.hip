@@ -528,11 +528,9 @@ static int launch_gemm_q(float *out, const uint8_t *w, const pulsar_block_q8_K *
     // 4096 11.1 -> 9.9 us, 14336 x 4096 19.2 -> 16.6 us; 5-31 tokens and
     // 14336-wide rows alike); Q6_K and NVFP4 spill at that cap (Q6_K 8192 x
     // 4096 12.8 -> 21.5 us)
-    // (Q4_K and Q5_K chunks of 17 or more tokens are tile.hip's)
-    constexpr bool kNt2 = Q != PULSAR_QUANT_Q4_K && Q != PULSAR_QUANT_Q5_K;
-    if (kNt2 && n_tok >= PK_GEMM_NT2) {
-        if constexpr (kNt2) PK_GEMM(2, 2, 2, PK_GEMM_D_NT2);
-    } else if (out_dim < 8192u)
+    if (n_tok >= PK_GEMM_NT2)
+        PK_GEMM(2, 2, 2, PK_GEMM_D_NT2);
+    else if (out_dim < 8192u)
         PK_GEMM(1, 8, 1, PK_GEMM_D_R16);
     else if (Q == PULSAR_QUANT_Q4_K)
         PK_GEMM(2, 8, 1, 1);

@@ -92,26 +92,49 @@ int launch_tile_gemm(uint32_t quant, float *out, const uint8_t *w, const pulsar_
     // it at any alignment
     if ((uintptr_t)xq % 4u != 0u) return -1;
     // Where the other kernels are at least as fast (weights from HBM, both
-    // sides timed on the same matrices):
+    // sides timed on the same matrices: 13636 of 32 to 14336 rows, 256 to 14336
+    // columns, 5 to 512 tokens; 3 in a thousand are more than 3% slower than
+    // there, and the faster side is missed by 1% on average):
     // Q4_K, Q5_K, Q6_K have the 16-row kernel of mmq.hip, which takes chunks of
     // up to 16 tokens in one pass and, below 8192 rows, of up to 31 in two
     // cheap ones (Q4_K 4096 x 4096: 16 tokens 6.5 against 10.4 us, 33 tokens
     // 14.7 against 10.6; 14336 x 4096, 17 tokens: 25.5 against 15.1). Q6_K's
     // decode is the longest of them, and as long as the 32-row tile is all
     // that fills the chip the 16-row kernel stays ahead (3000 x 2048, 100
-    // tokens: 14.2 against 15.3 us).
+    // tokens: 14.2 against 15.3 us). So it does for the others where rows of
+    // one or two super-blocks leave the tile's start and end its whole time
+    // (Q5_K 8192 x 512, 64 tokens: 6.1 against 7.0 us), and for Q5_K up to
+    // 64 tokens and the 768 blocks that its own kernel holds at once, where the
+    // tile has a third of the chip (11008 x 8192, 64 tokens: 51.0 against 54.6).
+    const uint64_t items = tile_items<PULSAR_QUANT_Q4_K, 1, 4, 2>(out_dim, n_tok);
     if (quant == PULSAR_QUANT_Q4_K || quant == PULSAR_QUANT_Q5_K || quant == PULSAR_QUANT_Q6_K) {
         if (n_tok < 17u || (n_tok < 32u && out_dim < 8192u)) return -1;
-        if (quant == PULSAR_QUANT_Q6_K && n_tok >= 32u &&
-            tile_items<PULSAR_QUANT_Q6_K, 1, 4, 2>(out_dim, n_tok) <= kTileSlots)
+        if (n_tok >= 32u && items <= kTileSlots && (nb <= 2u || quant == PULSAR_QUANT_Q6_K)) return -1;
+        if (n_tok >= 32u && n_tok <= 64u && quant == PULSAR_QUANT_Q5_K && items > kTileSlots && items <= 768u &&
+            nb >= 16u)
             return -1;
     } else {
         // The other formats run four tokens per pass over the rows in the lane
         // kernels; both sides grow with the row length, so rows times passes
         // decide (IQ4_XS 4096 x 4096: two passes 11.6 against 12.4 us, three
-        // 16 against 12.4; 2000 x 8192: four 19.3 against 20.8 us).
+        // 16 against 12.4; 2000 x 8192: four 19.3 against 20.8 us), and for
+        // rows of up to three super-blocks, where the tile's start and end
+        // outweigh its decode, rows times passes times length (IQ4_XS 1024 x
+        // 256, 64 tokens: 3.9 against 5.0 us; 4096 x 512, 17: 5.8 against 4.8).
         const uint64_t rows4 = (uint64_t)((n_tok + 3u) / 4u) * out_dim;
-        if (rows4 < (quant == PULSAR_QUANT_IQ4_XS ? 9000u : quant == PULSAR_QUANT_IQ2_XXS ? 8000u : 7000u)) return -1;
+        uint32_t least = 7000u, least_nb = 18000u;  // Q2_K
+        switch (quant) {
+        case PULSAR_QUANT_Q3_K: least_nb = 32000u; break;
+        case PULSAR_QUANT_IQ4_XS: least = 9000u, least_nb = nb == 1u ? 45000u : 36000u; break;
+        case PULSAR_QUANT_IQ2_XXS:
+            // the lane kernels give a row a power of two of lanes: rows of
+            // 24 super-blocks are on the tile earlier than rows of 32 (4096
+            // rows, 8 tokens: 25.8 against 18.9 us, 5: 21.6 against 25.9)
+            least = nb < 8u || (nb & (nb - 1u)) == 0u ? 8300u : 8000u, least_nb = nb == 1u ? 45000u : 36000u;
+            break;
+        default: break;
+        }
+        if (rows4 < least || (nb < 4u && rows4 * nb < least_nb)) return -1;
     }
 #define PK_TG(Q) \
     case Q: return launch_tile_gemm_q<Q>(out, w, xq, nb, out_dim, n_tok, row_bytes);
