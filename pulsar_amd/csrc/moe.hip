@@ -611,7 +611,7 @@ extern template int launch_grouped_mmq_kq<ExpertGroups>(bool, uint32_t, float *,
                                                         uint32_t, uint32_t, uint64_t, uint32_t, uint32_t);
 uint32_t grouped_mmq_pairs(bool pair, uint32_t quant, uint32_t k_dim, uint32_t lst_bytes);
 // tile_moe.hip: the grouped stages on the wide tile
-uint32_t tile_min_quarter_pairs(bool pair, uint32_t quant, uint32_t nb, uint32_t n_rows, uint32_t groups,
+uint32_t tile_min_quarter_pairs(bool csr, bool pair, uint32_t quant, uint32_t nb, uint32_t n_rows, uint32_t groups,
                                 uint32_t pmax);
 int launch_tile_experts(bool pair, uint32_t quant, float *out, const ExpertGroups &src, const float *weights,
                         const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
@@ -658,12 +658,13 @@ static int grouped_stage(bool pair, uint32_t quant, float *out, G grp, const flo
     // the tile's copies to LDS move whole dwords of act, which the other
     // kernels load at any alignment
     const bool fits = k_dim <= 16384u && (uintptr_t)act % 4u == 0u;
-    const uint32_t groups = std::is_same<G, ExpertGroups>::value ? sizes.experts : n_group;
-    const uint32_t bound = fits ? tile_min_quarter_pairs(pair, quant, k_dim / 256u, n_rows, groups,
+    constexpr bool kCsr = std::is_same<G, CsrGroups>::value;
+    const uint32_t bound = fits ? tile_min_quarter_pairs(kCsr, pair, quant, k_dim / 256u, n_rows,
+                                                         kCsr ? n_group : sizes.experts,
                                                          grouped_mmq_pairs(pair, quant, k_dim, lst_bytes))
                                 : 0u;
     if (bound == 0u) return mmq_or_lane(grp);
-    if constexpr (std::is_same<G, ExpertGroups>::value) {
+    if constexpr (!kCsr) {
         auto tile = [&](const ExpertGroups &src, uint32_t groups) {
             return launch_tile_experts(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, groups, row_bytes,
                                        act_op, lst_bytes);

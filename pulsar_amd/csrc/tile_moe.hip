@@ -175,42 +175,60 @@ __global__ __launch_bounds__(256, 2) void tile_csr_kernel(float *__restrict__ ou
 // row.
 //
 // The 16-row kernel reads an expert's weights once per pmax pairs, the tile once
-// per 64 with more work per super-block: a group of m pairs costs the one about
-// m / pmax + 1/2 passes and the other a fixed number of them, which grows with
-// the row length (a pass over a short row is mostly its staging) up to a bound.
-// That number, from 1400 stages of 10 layer shapes timed on both (8 to 256
-// experts, 2 to 56 super-blocks, 1 to 256 pairs per expert, weights from HBM),
-// in hundredths: none of them is more than 1% slower than on the 16-row kernel,
-// and the faster kernel is missed by 0.7% on average. Some of them:
-// gate / up, us by pairs per expert, 16-row / tile: IQ2_XXS 128 experts of 1536
-// x 4096, 4: 239 / 321, 6: 331 / 330, 12: 615 / 338; 32 of 2816 x 2816, 6: 82 /
-// 123, 10: 139 / 126; Q2_K 16 of 6400 x 4096, 4: 77 / 90, 8: 133 / 117; Q5_K 32
-// of 2816 x 2816, 5: 94 / 120, 8: 133 / 123; Q4_K 128 of 768 x 2048, 4: 74 / 70;
-// down, Q6_K 128 of 2048 x 768, 12: 88 / 97, 16: 112 / 100.
+// per 64 or 128 with more work per super-block: a group of m pairs costs the one
+// about m / pmax + 1/2 passes and the other a fixed number of them, which grows
+// with the row length (a pass over a short row is mostly its staging) up to a
+// bound. That number, in hundredths, is fitted to stages timed on both (10 layer
+// shapes of 8 to 256 experts, rows of 2 to 56 super-blocks, gate / up of 8 and
+// more, 1 to 400 pairs per expert, weights from HBM). It is lower for groups
+// found from the router's ids, which the 16-row kernel scans a wave at a time
+// before its passes, than for a CSR, where the tile is a launch of its own.
+//   router's ids, 1444 stages: none more than 1% slower than on the 16-row
+//   kernel, the faster kernel missed by 0.7% on average. us by pairs per expert,
+//   16-row / tile: gate / up IQ2_XXS 128 experts of 1536 x 4096, 4: 239 / 321,
+//   6: 331 / 330, 12: 615 / 338; 32 of 2816 x 2816, 6: 82 / 123, 10: 139 / 126;
+//   Q2_K 16 of 6400 x 4096, 4: 77 / 90, 8: 133 / 117; Q4_K 128 of 768 x 2048, 4:
+//   74 / 70; down Q6_K 128 of 2048 x 768, 12: 88 / 97, 16: 112 / 100.
+//   CSR, 2024 stages: 5 more than 3% slower (the worst 13%), the faster kernel
+//   missed by 0.1% on average. Gate / up Q4_K 128 of 768 x 2048, 7: 73 / 78, 8:
+//   85 / 79; Q2_K 128 of 1536 x 4096, 6: 205 / 225, 7: 231 / 227; IQ2_XXS, 7: 294 /
+//   349, 8: 364 / 352; down Q6_K 128 of 2048 x 768, 24: 105 / 109, 28: 115 / 111;
+//   Q4_K 256 of 2048 x 512, 12: 66 / 75, 16: 81 / 79.
 // Where a launch's blocks leave CUs idle the 16-row kernel's passes are one
-// after the other (8 experts of 2048 x 4096, IQ2_XXS, 4: 56 / 48).
+// after the other (router's ids, 8 experts of 2048 x 4096, IQ2_XXS, 4: 56 / 48).
 // Against the lane kernels the line lies at 2 to 3 pairs for the rows the
 // 16-row kernel cannot hold (8 experts of 4096 x 14336, down, lane / tile, 2:
 // Q6_K 216 / 188, Q4_K 169 / 103, IQ2_XXS 119 / 163; 3: IQ2_XXS 179 / 164) and
-// at 1.5 for Q3_K and IQ4_XS (IQ4_XS 128 of 768 x 2048, 1: 51 / 57, 1.5: 89 /
-// 72), whose down stages of one or two super-blocks reach it at 2.
-uint32_t tile_min_quarter_pairs(bool pair, uint32_t quant, uint32_t nb, uint32_t n_rows, uint32_t groups,
+// at 1.5 (CSR: 2) for Q3_K and IQ4_XS (router's ids, IQ4_XS 128 of 768 x 2048,
+// 1: 51 / 57, 1.5: 89 / 72), half a pair later in down stages of one or two
+// super-blocks.
+uint32_t tile_min_quarter_pairs(bool csr, bool pair, uint32_t quant, uint32_t nb, uint32_t n_rows, uint32_t groups,
                                 uint32_t pmax) {
     struct Passes {
         uint32_t base, per_sb, most;
     } p;
     switch (quant) {
-    case PULSAR_QUANT_Q4_K: p = pair ? Passes{70, 5, 150} : Passes{45, 10, 160}; break;
-    case PULSAR_QUANT_Q5_K: p = pair ? Passes{93, 5, 180} : Passes{68, 13, 170}; break;
-    case PULSAR_QUANT_Q6_K: p = pair ? Passes{100, 8, 220} : Passes{90, 15, 290}; break;
-    case PULSAR_QUANT_Q2_K: p = pair ? Passes{84, 6, 180} : Passes{65, 13, 170}; break;
-    case PULSAR_QUANT_IQ2_XXS: p = pair ? Passes{90, 10, 260} : Passes{120, 15, 240}; break;
+    case PULSAR_QUANT_Q4_K:
+        p = csr ? pair ? Passes{45, 10, 150} : Passes{125, 2, 150} : pair ? Passes{70, 5, 150} : Passes{45, 10, 160};
+        break;
+    case PULSAR_QUANT_Q5_K:
+        p = csr ? pair ? Passes{45, 10, 170} : Passes{140, 6, 170} : pair ? Passes{93, 5, 180} : Passes{68, 13, 170};
+        break;
+    case PULSAR_QUANT_Q6_K:
+        p = csr ? pair ? Passes{40, 18, 230} : Passes{195, 4, 280} : pair ? Passes{100, 8, 220} : Passes{90, 15, 290};
+        break;
+    case PULSAR_QUANT_Q2_K:
+        p = csr ? pair ? Passes{125, 4, 210} : Passes{150, 2, 170} : pair ? Passes{84, 6, 180} : Passes{65, 13, 170};
+        break;
+    case PULSAR_QUANT_IQ2_XXS:
+        p = csr ? pair ? Passes{130, 6, 280} : Passes{145, 28, 230} : pair ? Passes{90, 10, 260} : Passes{120, 15, 240};
+        break;
     case PULSAR_QUANT_Q3_K:
-    case PULSAR_QUANT_IQ4_XS: return !pair && nb <= 2u ? 8u : 6u;
+    case PULSAR_QUANT_IQ4_XS: return (csr ? 8u : 6u) + (!pair && nb <= 2u ? 2u : 0u);
     default: return 0u;
     }
     if (pmax == 0u) return quant == PULSAR_QUANT_IQ2_XXS ? 12u : 8u;
-    uint32_t passes = p.base + p.per_sb * nb;
+    uint32_t passes = p.base + p.per_sb * (pair && nb < 8u ? 8u : nb);
     if (passes > p.most) passes = p.most;
     const uint32_t rows = pair ? 64u : 128u;
     if (quant != PULSAR_QUANT_Q6_K && (uint64_t)((n_rows + rows - 1u) / rows) * groups <= 256u && passes > 130u)

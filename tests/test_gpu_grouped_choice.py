@@ -250,3 +250,27 @@ def test_choice_by_measured_crossover(dev, stage):
     nodes = launches(call)
     assert len(nodes) == 1
     assert (nodes[0].shared == 4 * T * k) == (stage in ON_TILE)
+
+
+@pytest.mark.parametrize("stage", [
+    # format, down, groups, rows, cols, the most pairs per group short of the line and the least past it
+    (QUANT_Q4_K, False, 128, 768, 2048, 7, 8), (QUANT_Q2_K, False, 128, 1536, 4096, 6, 8),
+    (QUANT_IQ2_XXS, False, 128, 1536, 4096, 7, 9), (QUANT_Q6_K, True, 128, 2048, 768, 24, 28),
+    (QUANT_Q4_K, True, 256, 2048, 512, 12, 16), (QUANT_IQ4_XS, True, 256, 2048, 512, 2, 3)],
+    ids=lambda s: "-".join(map(str, s)))
+def test_csr_choice_by_measured_crossover(dev, stage):
+    """A CSR that can hold groups past the line takes the tile's launch too, one
+    short of it does not (recorded, not run)."""
+    quant, down, groups, rows, cols, under, over = stage
+    buf = torch.zeros(256, dtype=torch.uint8, device=dev)
+    for per_group, want in ((under, 1), (over, 2)):
+        pairs = torch.zeros(per_group * groups, dtype=torch.int32, device=dev)
+
+        def call():
+            if down:
+                K.moe_down_grouped(buf, buf, buf, pairs, buf, cols, rows, 8, groups, row_bytes(quant, cols), quant)
+            else:
+                K.moe_pair_swiglu_grouped(buf, buf, buf, pairs, buf, buf, cols, rows, 8, groups, row_bytes(quant, cols),
+                                          quant, 0)
+
+        assert len(launches(call)) == want
