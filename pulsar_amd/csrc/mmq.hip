@@ -758,6 +758,7 @@ __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_e
         float *__restrict__ out, const G src, const float *__restrict__ weights,
         const pulsar_block_q8_K *__restrict__ act, uint32_t k_blocks, uint32_t lim, uint32_t n_rows,
         uint32_t n_used, uint64_t row_bytes, uint32_t act_op, uint32_t pmax, uint32_t lst_off) {
+    if (src.tiled()) return;  // a caller's CSR whose groups are long on average: before any other work
     using F = GmmqFmt<Q>;
     constexpr uint32_t NM = PAIR ? 2 : 1;
     constexpr bool kIq2 = Q == PULSAR_QUANT_IQ2_XXS;
@@ -784,7 +785,6 @@ __global__ __launch_bounds__(64 * kGqWaves<Q>) __attribute__((amdgpu_waves_per_e
     }
     const uint32_t group = blockIdx.y;
     const typename G::Group grp = src.group(group);
-    if (src.tiled()) return;  // a caller's CSR whose groups are long on average
     const pulsar_expert_ptrs &p = grp.p;
     const uint8_t *w0 = PAIR ? (const uint8_t *)p.gate : (const uint8_t *)p.down;
     const uint8_t *w1 = PAIR ? (const uint8_t *)p.up : nullptr;

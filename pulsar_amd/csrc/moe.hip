@@ -164,6 +164,7 @@ __global__ __launch_bounds__(256) void moe_pair_grouped_kernel(
         const pulsar_block_q8_K *__restrict__ xq, uint32_t n_units, uint32_t nblk32, uint32_t lpr_log2,
         uint32_t in_blocks, uint32_t mid_dim, uint32_t n_used, uint64_t row_bytes, uint32_t act_op, uint32_t pmax,
         uint32_t lst_off) {
+    if (grp.tiled()) return;
     PK_FMT_LUT(Q)
     extern __shared__ __align__(16) uint8_t acts_lds[];
     __shared__ uint32_t pr_l[kGrpMaxPairs];
@@ -172,7 +173,6 @@ __global__ __launch_bounds__(256) void moe_pair_grouped_kernel(
     const pulsar_expert_ptrs &p = gr.p;
     const bool nul = gr.is_null();
     if (!nul && (!p.gate || !p.up)) return;
-    if (grp.tiled()) return;
     uint32_t *lst = (uint32_t *)(acts_lds + lst_off);
     uint32_t s0, s1;
     grp.range(gr, lst, s0, s1);
@@ -249,6 +249,7 @@ __global__ __launch_bounds__(256) void moe_down_grouped_kernel(
         float *__restrict__ partial, const G grp, const pulsar_block_q8_K *__restrict__ midq, uint32_t n_units,
         uint32_t nblk32, uint32_t lpr_log2, uint32_t mid_blocks, uint32_t out_dim, uint32_t n_used,
         uint64_t row_bytes, uint32_t pmax, uint32_t lst_off) {
+    if (grp.tiled()) return;
     PK_FMT_LUT(Q)
     extern __shared__ __align__(16) uint8_t acts_lds[];
     __shared__ uint32_t pr_l[kGrpMaxPairs];
@@ -257,7 +258,6 @@ __global__ __launch_bounds__(256) void moe_down_grouped_kernel(
     const pulsar_expert_ptrs &p = gr.p;
     const bool nul = gr.is_null();
     if (!nul && !p.down) return;
-    if (grp.tiled()) return;
     uint32_t *lst = (uint32_t *)(acts_lds + lst_off);
     uint32_t s0, s1;
     grp.range(gr, lst, s0, s1);

@@ -212,7 +212,7 @@ uint32_t tile_min_quarter_pairs(bool csr, bool pair, uint32_t quant, uint32_t nb
         p = csr ? pair ? Passes{45, 10, 150} : Passes{125, 2, 150} : pair ? Passes{70, 5, 150} : Passes{45, 10, 160};
         break;
     case PULSAR_QUANT_Q5_K:
-        p = csr ? pair ? Passes{45, 10, 170} : Passes{140, 6, 170} : pair ? Passes{93, 5, 180} : Passes{68, 13, 170};
+        p = csr ? pair ? Passes{60, 10, 170} : Passes{140, 6, 170} : pair ? Passes{93, 5, 180} : Passes{68, 13, 170};
         break;
     case PULSAR_QUANT_Q6_K:
         p = csr ? pair ? Passes{40, 18, 230} : Passes{195, 4, 280} : pair ? Passes{100, 8, 220} : Passes{90, 15, 290};
