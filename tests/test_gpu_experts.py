@@ -3,7 +3,8 @@ quantize -> moe_down_experts) against the CSR path it replaces
 (moe_route_group -> moe_pair_swiglu_grouped -> quantize ->
 moe_down_grouped, itself checked against the oracle in test_gpu_moe.py and
 test_gpu_fullsize.py): routing outputs, every mid row and every partial row
-bit-identical, unrouted slots written as 0."""
+bit-identical, unrouted slots written as 0. (Where the two choose different
+kernels: test_gpu_grouped_choice.py.)"""
 import numpy as np
 import pytest
 import torch
@@ -152,7 +153,8 @@ CASES = [
     (QUANT_Q4_K, QUANT_Q6_K, 512, 256, 96, 8, 20, 1, 1, ACT_SILU, False),
     (fm.QUANT_Q5_K, fm.QUANT_Q5_K, 512, 512, 16, 4, 9, 0, 0, ACT_SILU, False),
     (QUANT_MXFP4, QUANT_MXFP4, 576, 320, 8, 4, 64, 0, 1, ACT_SWIGLU_OAI, True),
-    # lane kernels (formats without a matrix-core grouped kernel)
+    # formats without a 16-row kernel: here on the wide tile, with shorter groups
+    # on the lane kernels; and two that only the lane kernels have
     (fm.QUANT_Q3_K, fm.QUANT_IQ4_XS, 512, 256, 10, 3, 7, 1, 1, ACT_SILU, True),
     (fm.QUANT_Q8_0, fm.QUANT_IQ2_S, 256, 512, 6, 2, 5, 0, 0, ACT_SWIGLU_OAI, False),
 ]

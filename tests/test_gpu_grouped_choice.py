@@ -274,3 +274,181 @@ def test_csr_choice_by_measured_crossover(dev, stage):
                                           quant, 0)
 
         assert len(launches(call)) == want
+
+
+# ------------------------------------------ the tile's branches, on the oracle
+
+@pytest.mark.parametrize("act", [fm.ACT_SILU, fm.ACT_SWIGLU_OAI])
+@pytest.mark.parametrize("quant", [QUANT_Q4_K, QUANT_Q2_K, QUANT_Q6_K, QUANT_IQ4_XS], ids=lambda q: fm.NAMES[q])
+def test_tile_biases_and_activation(dev, quant, act):
+    """Gate and up biases (one expert without) and both activations on the tile,
+    from both sources, against the oracle's dots."""
+    sizes = [70, 33, 40]
+    s = Stage(dev, quant, False, sizes, 512, 200)
+    rng = np.random.default_rng(act)
+    bias = [rng.standard_normal((s.E, s.rows)).astype(np.float32) for _ in range(2)]
+    d_bias = [torch.from_numpy(b).to(dev) for b in bias]
+    order = list(range(s.E))
+    _, starts, pairs = s.csr_arrays(order)
+    g = K.expert_ptrs([s.entry(e) + tuple(b.data_ptr() + 4 * e * s.rows if e != 1 else 0 for b in d_bias)
+                       for e in order])
+    csr = s.zeros()
+    K.moe_pair_swiglu_grouped(csr, up(g), up(starts), up(pairs), s.d_w, s.d_xq, s.cols, s.rows, s.n_used, s.E, s.rb,
+                              quant, act)
+    got = {"csr": down_np(csr)}
+    p = [m.data_ptr() for m in s.d_mats]
+    active = np.array([s.E, int((s.ids == -1).sum())] + order, np.uint32)
+    bank = K.ExpertBank(p[0], p[1], None, d_bias[0].data_ptr(), d_bias[1].data_ptr(), None, s.step, s.step, 0, s.rows,
+                        s.rows, 0)
+    exp = s.zeros()
+    K.moe_pair_swiglu_experts(exp, up(s.ids), up(active), s.d_w, s.d_xq, bank, s.E, [], s.T, s.n_used, s.cols, s.rows,
+                              s.rb, quant, act)
+    got["experts"] = down_np(exp)
+    flat = s.ids.reshape(-1)
+    for e in order:
+        at = np.flatnonzero(flat == e)
+        (gv, _, bg), (uv, _, bu) = (rows_want(quant, m[e], s.rb, s.xq[at // s.n_used], s.cols, at.size) for m in s.mats)
+        gv, uv, bg, bu = (v.astype(np.float64) for v in (gv, uv, 1e-5 * bg, 1e-5 * bu))
+        w = s.wts.reshape(-1)[at].astype(np.float64)[:, None]
+        for who, rows in got.items():
+            g0, u0, eg, eu = gv, uv, bg, bu
+            if e != 1 or who == "experts":  # the bank gives every expert its biases
+                g0, u0 = gv + bias[0][e], uv + bias[1][e]
+                eg, eu = bg + 2.0**-24 * np.abs(g0), bu + 2.0**-24 * np.abs(u0)
+            if act == fm.ACT_SWIGLU_OAI:  # the clamps spread no error; sigmoid sharpened by 1.702
+                g1 = np.minimum(g0, 7.0)
+                a, f = g1 / (1 + np.exp(-1.702 * g1)), np.clip(u0, -7, 7) + 1
+            else:
+                a, f = g0 / (1 + np.exp(-g0)), u0
+            # |(g sigmoid(k g))'| <= 1.1 for either k; exp, division and products: 1e-6
+            bound = w * (1.1 * eg * (np.abs(f) + eu) + np.abs(a) * eu) + 1e-6 * np.abs(a * f) * w + 1e-30
+            err = np.abs(rows[at] - a * f * w)
+            assert (err <= bound).all(), (who, e, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("down", [False, True])
+@pytest.mark.parametrize("quant", [QUANT_Q4_K, QUANT_Q6_K, QUANT_Q3_K], ids=lambda q: fm.NAMES[q])
+def test_tile_csr_forms(dev, quant, down):
+    """CSRs the device-built ones never are: pairs that start past the first
+    entry, empty groups between full ones, a group with pairs and NULL pointers
+    (its rows stay untouched)."""
+    sizes = [40, 0, 65, 1, 0, 130]
+    s = Stage(dev, quant, down, sizes, *((200, 512) if down else (512, 200)))
+    whole = s.run_csr(s.csr_arrays())
+    s.check(whole, "csr")
+    order = [-1, 0, 1, -1, -1, 2, 3, 4, 5, -1]
+    assert np.array_equal(s.run_csr(s.csr_arrays(order, skip=37)).view(np.uint32), whole.view(np.uint32))
+    g, starts, pairs = s.csr_arrays()
+    g[2] = 0
+    got, null = s.run_csr((g, starts, pairs)), s.ids.reshape(-1) == 2
+    assert not got[null].any()
+    assert np.array_equal(got[~null].view(np.uint32), whole[~null].view(np.uint32))
+
+
+@pytest.mark.parametrize("quant", [QUANT_Q4_K, QUANT_Q3_K], ids=lambda q: fm.NAMES[q])
+@pytest.mark.parametrize("groups", [1023, 1024, 1025])
+def test_csr_of_many_groups(dev, quant, groups):
+    """The tile counts the tiles of up to 1024 groups; a CSR of more stays on the
+    kernels without that limit. 12 pairs per group, 8 matrices."""
+    s = Stage(dev, quant, False, [12] * 8, 512, 64)
+    order = np.arange(groups) % s.E
+    g, starts, pairs = s.csr_arrays()
+    lists = [pairs[starts[e]:starts[e + 1]] for e in range(s.E)]
+    arrays = (g[order], (12 * np.arange(groups + 1)).astype(np.uint32), np.concatenate([lists[e] for e in order]))
+    out, dev_arrays = s.zeros(), [up(a) for a in arrays]
+    n = len(launches(lambda: s.queue_csr(dev_arrays, groups, out)))
+    assert n == (1 if groups > 1024 else 2)
+    s.check(s.run_csr(arrays), "csr")
+
+
+def test_skewed_groups_on_the_16_row_kernel(dev):
+    """One long group among many single pairs: the mean keeps the stage on the
+    16-row kernel, which walks the long one in several pair tiles; the same rows
+    as where that group is alone and long enough for the tile."""
+    for quant in ROW16:
+        for down in (False, True):
+            s = Stage(dev, quant, down, [150] + [1] * 199, *((77, 512) if down else (512, 77)), n_used=2)
+            both = s.run_csr(s.csr_arrays())
+            s.check(both, "skewed")
+            alone, at = s.run_csr(s.csr_arrays([0])), s.ids.reshape(-1) == 0
+            assert np.array_equal(both[at].view(np.uint32), alone[at].view(np.uint32)), (fm.NAMES[quant], down)
+
+
+@pytest.mark.parametrize("quant", [QUANT_Q4_K, QUANT_Q2_K, QUANT_Q6_K], ids=lambda q: fm.NAMES[q])
+@pytest.mark.parametrize("n_tok", [33, 128])
+def test_shared_slot_equal_from_both_sources(dev, quant, n_tok):
+    """Few pairs per routed expert and a shared slot of every token: from the
+    router's ids the shared group is a launch of its own on the tile (gate / up
+    from 33 tokens, down from 100), in a CSR one group among the others."""
+    E, k = 256, 2
+    for down in (False, True):
+        sizes = [1] * E + [n_tok]
+        s = Stage(dev, quant, down, sizes, *((140, 512) if down else (512, 140)), n_used=3)
+        rng = np.random.default_rng(n_tok)
+        ids = np.stack([np.append(rng.choice(E, k, replace=False), E) for _ in range(n_tok)]).astype(np.int32)
+        s.ids, s.T = ids, n_tok
+        s.xq = oracle.quantize_q8_k(rng.standard_normal((n_tok * (3 if down else 1), s.cols)).astype(np.float32) * 1e-2)
+        s.wts = np.concatenate([rng.uniform(0.1, 1, (n_tok, k)), np.ones((n_tok, 1))], 1).astype(np.float32)
+        s.d_xq, s.d_w = up(s.xq), torch.from_numpy(s.wts).to(dev)
+        csr = s.run_csr(s.csr_arrays())
+        s.check(csr, "csr")
+        first = list(dict.fromkeys(int(e) for e in ids[:, :k].reshape(-1)))
+        active = np.zeros(2 + E, np.uint32)
+        active[:2 + len(first)] = [len(first), 0] + first
+        p = [m.data_ptr() for m in s.d_mats]
+        out, args = s.zeros(), (up(np.ascontiguousarray(ids[:, :k])), up(active))
+        if down:
+            bank = K.ExpertBank(None, None, p[0], None, None, None, 0, 0, s.step, 0, 0, 0)
+            call = lambda: K.moe_down_experts(out, *args, s.d_xq, bank, E, [s.entry(E)], n_tok, k, s.cols, s.rows, s.rb,
+                                              quant)
+        else:
+            bank = K.ExpertBank(p[0], p[1], None, None, None, None, s.step, s.step, 0, 0, 0, 0)
+            call = lambda: K.moe_pair_swiglu_experts(out, *args, s.d_w, s.d_xq, bank, E, [s.entry(E)], n_tok, k, s.cols,
+                                                     s.rows, s.rb, quant, 0)
+        assert len(launches(call)) == (2 if not down or n_tok >= 100 else 1)
+        call()
+        assert np.array_equal(down_np(out).view(np.uint32), csr.view(np.uint32)), down
+
+
+@pytest.mark.parametrize("down", [False, True])
+def test_tile_of_2048_ids(dev, down):
+    """The most ids a block scans: 2048, a quarter to each wave, 8 strips of 64."""
+    s = Stage(dev, QUANT_Q4_K, down, [300, 700, 1, 450, 585], *((70, 512) if down else (512, 70)), n_used=4)
+    assert s.ids.size == 2048  # 12 of them route nowhere
+    got = s.run_experts()
+    s.check(got, "experts")
+    assert not got[s.ids.reshape(-1) == -1].any()
+
+
+@pytest.mark.parametrize("quant,down", [(QUANT_Q4_K, False), (QUANT_Q6_K, True), (QUANT_Q3_K, False)])
+def test_csr_graph_follows_the_group_sizes(dev, quant, down):
+    """A CSR stage captured once, its arrays replaced between replays: short,
+    long, short and unevenly long groups take their kernel inside the same graph,
+    and every replay equals an eager run."""
+    E = 24
+    s = Stage(dev, quant, down, [40] * E, *((140, 512) if down else (512, 140)))
+    flat = s.ids.reshape(-1)
+    cap, out = up(np.zeros(flat.size, np.uint32)), s.zeros()
+    g, starts = up(s.csr_arrays()[0]), up(np.zeros(E + 1, np.uint32))
+    call = lambda: s.queue_csr((g, starts, cap), E, out)
+    graph = runtime.Graph.capture(call)
+    for per in ([1] * E, [40] * E, [2] * E, [40] * 3 + [1] * (E - 3), [0] * (E - 1) + [40], [40] * E):
+        lists = [np.flatnonzero(flat == e)[:n] for e, n in enumerate(per)]
+        i = np.concatenate(lists)
+        pairs = np.zeros(flat.size, np.uint32)
+        pairs[:i.size] = i // s.n_used << 4 | i % s.n_used
+        cap.copy_(up(pairs))
+        starts.copy_(up(np.concatenate([[0], np.cumsum([len(v) for v in lists])]).astype(np.uint32)))
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.launch()
+        runtime.sync()
+        replay = down_np(out).copy()
+        out.zero_()
+        torch.cuda.synchronize()
+        call()
+        runtime.sync()
+        assert np.array_equal(replay.view(np.uint32), down_np(out).view(np.uint32)), per
+        listed = np.zeros(flat.size, bool)
+        listed[i] = True
+        assert replay[listed].any(1).all() and not replay[~listed].any()

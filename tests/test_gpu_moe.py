@@ -286,10 +286,12 @@ def test_grouped_random_shapes(dev, q, hidden, ffn, E, n_used, n_tok, nulls, see
                                           (QUANT_Q4_K, 512, 512), (fm.QUANT_Q5_K, 256, 512),
                                           (QUANT_Q6_K, 512, 256), (QUANT_MXFP4, 1280, 416)])
 def test_grouped_many_pairs_per_expert(dev, q, hidden, ffn):
-    """Groups of 20-39 pairs (two or three pair tiles per weight pass) over
-    matrices of several row tiles per wave: each pair tile walks the wave's
-    row tiles again from the first. 40 tokens x 2 slots over 3 experts, one
-    NULL slot."""
+    """Groups of 20-39 pairs over matrices of several row tiles per wave. 40
+    tokens x 2 slots over 3 experts, one NULL slot. Stages whose groups are long
+    enough run on the wide tile, MXFP4 and the others on the 16-row kernel, where
+    each pair tile (two or three per weight pass) walks the wave's row tiles again
+    from the first; test_gpu_grouped_choice.py has such groups on the 16-row
+    kernel for every format of it."""
     L = Layer(q, q, hidden=hidden, ffn=ffn, E=3, n_used=2, n_tok=40, biases=q == QUANT_MXFP4, seed=5)
     L.sel[:, 0] = 0
     L.sel[:, 1] = np.where(np.arange(40) % 2 == 0, 1, 2)
@@ -607,8 +609,9 @@ def test_library_selftests(dev):
 
 
 def test_grouped_wide_rows_lane_fallback(dev):
-    """Rows too wide for the MFMA kernel's staged activations (14336 values:
-    56 q8_K blocks per pair > the 16 KiB tile) run the grouped lane kernels."""
+    """Rows of 14336 values, of which a gate / up tile of the 16-row kernel holds
+    one pair (two pairs per group: the wide tile). Down rows of that width, which
+    only the lane kernels and the tile hold: test_gpu_grouped_choice.py."""
     L = Layer(QUANT_Q4_K, QUANT_Q6_K, hidden=14336, ffn=256, E=3, n_used=2, n_tok=3)
     hptrs, dptrs = L.ptrs()
     xq = oracle.quantize_q8_k(L.x)
@@ -639,8 +642,9 @@ def test_pair_down_every_format(dev, q):
 
 @pytest.mark.parametrize("q", NEW_FORMATS, ids=lambda q: fm.NAMES[q])
 def test_grouped_every_format(dev, q):
-    """The same formats through the grouped entry points (Q5_K on the matrix
-    cores, the rest on the lane kernels)."""
+    """The same formats through the grouped entry points (Q5_K, Q3_K and IQ4_XS on
+    the matrix cores, the rest on the lane kernels; short groups of Q3_K and
+    IQ4_XS, which the lane kernels run: test_gpu_grouped_choice.py)."""
     L = Layer(q, q, hidden=512, ffn=256, E=5, n_used=4, n_tok=12, null_slots=(7,))
     hptrs, dptrs = L.ptrs()
     xq = oracle.quantize_q8_k(L.x)

@@ -184,8 +184,7 @@ def test_tile_grouped(dev, quant, down):
     exp = down_np(got)
     check_grouped(quant, mats, ids, xq, wts, exp, down, cols, "experts")
     assert not exp[np.flatnonzero(ids.reshape(-1) == -1)].any()  # NULL slots: rows of 0
-    if quant not in (QUANT_Q6_K,) or not down:  # both on the tile: the same sums
-        assert np.array_equal(csr, exp)
+    assert np.array_equal(csr, exp)  # both on the tile: the same sums
 
 
 def test_tile_shared_slot(dev):
