@@ -104,7 +104,8 @@ int pulsar_quantize_q8_K(void *out, const void *x, uint32_t in_dim, uint32_t n_r
  * IQ2_XXS, Q4_K, Q5_K, Q6_K, Q3_K, IQ4_XS, IQ4_NL, NVFP4 (the expert-only
  * formats return 0, as there); in_dim % 256 == 0. Chunks of 5 or more tokens
  * run on the int8 matrix cores (IQ4_NL and the smallest chunks of the formats
- * without a 16-row kernel excepted).
+ * without a 16-row kernel excepted). xq may start at any byte, here and in the
+ * grouped stages; rows on a 4-byte boundary run fastest.
  * Replaces pulsar_matmul_kq (pulsar_kernels.cu:4895). */
 int pulsar_matmul_kq(void *out, const void *w, const void *xq, uint32_t in_dim,
                      uint32_t out_dim, uint32_t n_tok, uint64_t row_bytes,

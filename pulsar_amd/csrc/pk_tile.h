@@ -609,8 +609,8 @@ constexpr uint32_t kTileSlots = 512;
 // addresses, two registers each, in every iteration: half the spills. Prefill
 // of 128 Q4_K / Q6_K experts, 1536 tokens top-8: 437 -> 401 us a layer; IQ2_XXS
 // chunk of 100 tokens: 498 -> 485. The 16-row kernel's fp32 step, which has three
-// more vector operations for formats with mins, takes that layer from 397 to
-// 404. The dense kernel keeps Tile::run: fixed in
+// more vector operations for formats with mins, takes the Q4_K stage of that
+// layer from 210 to 220 (the layer 400 -> 411). The dense kernel keeps Tile::run: fixed in
 // this order its 8-slice Q4_K tile spills 37 registers (77 -> 91 us), and its
 // tiles of 2 to 4 slices take 1-2% longer.
 template <uint32_t Q, uint32_t NS>

@@ -4,9 +4,10 @@
 //     the lane kernels), weights from HBM: Q4_K 14336 x 4096, 512 tokens 183 ->
 //     76 us (0.79 P int8-op/s), 1024 tokens 369 -> 153; IQ4_XS 8192 x 2816, 250
 //     tokens 372 -> 27; Q2_K 14336 x 4096, 512 tokens 1137 -> 60. What bounds it
-//     (counters, Q4_K, 512 tokens): matrix cores busy 35% of the time, vector
-//     units 35%, L1 lookups 44%; its 256 registers leave two waves per SIMD,
-//     which overlap these only in part.
+//     (counters, Q4_K, 512 tokens): vector units busy 42% of the time, matrix
+//     cores 34%; its 256 registers leave two waves per SIMD, which overlap
+//     these only in part: 30% of a wave's time waits for LDS and memory, 30%
+//     for an issue slot.
 #include "pk_tile.h"
 
 namespace pk {
