@@ -288,10 +288,10 @@ int pulsar_moe_route(void *selected, void *weights, void *ptrs, void *slot_weigh
  * pulsar_moe_pair_swiglu_grouped / pulsar_moe_down_grouped would for the
  * same pairs, so the rows they write are bit-identical to those calls',
  * whatever the sizes of the groups. One exception: stages that the lane
- * kernels run where groups are short (Q3_K, IQ4_XS; rows too wide for the
- * 16-row kernel's staged activations) equal them bit for bit where both
- * calls' groups have the same mean size (else their super-blocks are added
- * in another order).
+ * kernels run where groups are short (Q3_K, IQ4_XS: below about 2 pairs per
+ * group; rows of more than 13568 values: below 2 to 3). Each call goes by its
+ * own groups' mean; where one is short and the other is not, a row's
+ * super-blocks are added in another order and its last bits may differ.
  * Slots whose id is outside [0, n_expert) get rows of 0 in mid (partial),
  * so every row of mid [n_tok][k_used + n_shared][mid_dim] (partial
  * [..][out_dim]) is written and partial needs no zeroing. slot_weights

@@ -207,7 +207,7 @@ def moe_pair_swiglu_experts(mid, selected, active, slot_weights, xq, bank: "Expe
     """The grouped gate/up stage with one group per selected expert, grouped
     on the device from moe_route's outputs (rows equal
     moe_pair_swiglu_grouped's, for Q3_K, IQ4_XS and very wide rows where both
-    have groups of the same mean size; unrouted slots get rows of 0)."""
+    have short groups or neither has; unrouted slots get rows of 0)."""
     arr, n_shared = _shared_array(shared)
     _check(_lib.load().pulsar_moe_pair_swiglu_experts(
         _ptr(mid), _ptr(selected), _ptr(active), _ptr(slot_weights), _ptr(xq), ctypes.byref(bank), n_expert,
