@@ -615,7 +615,7 @@ uint32_t tile_min_quarter_pairs(bool csr, bool pair, uint32_t quant, uint32_t nb
                                 uint32_t pmax);
 int launch_tile_experts(bool pair, uint32_t quant, float *out, const ExpertGroups &src, const float *weights,
                         const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
-                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes);
+                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes, bool shared_only);
 int launch_tile_csr(bool pair, uint32_t quant, float *out, const CsrGroups &src, const float *weights,
                     const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
                     uint64_t row_bytes, uint32_t act_op);
@@ -665,19 +665,17 @@ static int grouped_stage(bool pair, uint32_t quant, float *out, G grp, const flo
                                 : 0u;
     if (bound == 0u) return mmq_or_lane(grp);
     if constexpr (!kCsr) {
-        auto tile = [&](const ExpertGroups &src, uint32_t groups) {
-            return launch_tile_experts(pair, quant, out, src, weights, act, k_dim, n_rows, n_used, groups, row_bytes,
-                                       act_op, lst_bytes);
+        auto tile = [&](uint32_t groups, bool shared_only) {
+            return launch_tile_experts(pair, quant, out, grp, weights, act, k_dim, n_rows, n_used, groups, row_bytes,
+                                       act_op, lst_bytes, shared_only);
         };
-        if (4u * sizes.pairs >= bound * sizes.experts) return tile(grp, n_group);
+        if (4u * sizes.pairs >= bound * sizes.experts) return tile(n_group, false);
         if (grp.n_shared != 0u && grp.n_tok >= (pair ? 33u : 100u)) {
-            G part = grp;
-            part.which = ExpertGroups::kRouted;
-            const int r = mmq(part);
+            G routed = grp;
+            routed.n_shared = 0u;  // their rows are the second launch's
+            const int r = mmq(routed);
             if (r < 0) return lane(grp);
-            if (r == 0) return r;
-            part.which = ExpertGroups::kShared;
-            return tile(part, grp.n_shared);
+            return r == 0 ? r : tile(grp.n_shared, true);
         }
         return mmq_or_lane(grp);
     } else {

@@ -325,10 +325,10 @@ PK_DEV SlotRoute route_slot(const float *lg, const float *rbias, uint32_t n_expe
 // pairs (token << 4 | slot, in pair order) through pair(), which a thread
 // may call for any index in [b, e) right after range().
 
-// The reference's grouped contract: a CSR by expert from the caller
-// (gptrs [n_group], starts [n_group + 1], pairs), pulsar_kernels.cu:3483-3591.
 constexpr uint32_t kCsrGroups = 1024;  // most groups whose tile counts a block of the wide tile keeps
 
+// The reference's grouped contract: a CSR by expert from the caller
+// (gptrs [n_group], starts [n_group + 1], pairs), pulsar_kernels.cu:3483-3591.
 struct CsrGroups {
     const pulsar_expert_ptrs *gptrs;
     const uint32_t *starts;
@@ -375,9 +375,6 @@ struct ExpertGroups {
     pulsar_expert_bank bank;
     SharedSlots shared;
     uint32_t n_expert, k_used, n_shared, n_tok;
-    // which groups a launch is for: all, all but the shared slots' (empty
-    // here), or the shared slots' alone (group g is shared slot g)
-    enum Part : uint32_t { kAll, kRouted, kShared } which;
     struct Group {
         pulsar_expert_ptrs p;
         uint32_t kind, e;  // kind 0: routed expert e, 1: shared slot e, 2: NULL, 3: empty
@@ -397,21 +394,25 @@ struct ExpertGroups {
         G.pf[1] = sel[lane + 64u < total ? lane + 64u : total - 1u];
         G.p = pulsar_expert_ptrs{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
         G.e = 0u;
-        if (which == kShared) {
-            G.kind = 1u;
-            G.e = g;
-            G.p = shared.p[g];
-        } else if (g < n_act) {
+        if (g < n_act) {
             G.kind = 0u;
             G.e = e_g;
             G.p = bank_ptrs(bank, n_expert, (int32_t)e_g);
         } else if (g < n_act + n_shared) {
-            G.kind = which == kRouted ? 3u : 1u;
+            G.kind = 1u;
             G.e = g - n_act;
             G.p = shared.p[G.e];
         } else {
             G.kind = g == n_act + n_shared && n_nul != 0u ? 2u : 3u;
         }
+        return G;
+    }
+    // Shared slot i's group, for a launch on the shared slots alone
+    PK_DEV Group shared_group(uint32_t i) const {
+        Group G = {};
+        G.kind = 1u;
+        G.e = i;
+        G.p = shared.p[i];
         return G;
     }
     // Every wave scans the selected ids and writes the same list to lst

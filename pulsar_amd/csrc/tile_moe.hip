@@ -70,19 +70,20 @@ struct GroupTile {
 };
 
 // Groups found from the router's ids: block = (row block, group), the group's
-// pairs in tiles of 16 NS one after the other.
+// pairs in tiles of 16 NS one after the other. shared_only: the groups are the
+// shared slots' alone.
 template <uint32_t Q, bool PAIR, uint32_t NS>
 __global__ __launch_bounds__(256, 2) void tile_experts_kernel(float *__restrict__ out, const ExpertGroups src,
                                                               const float *__restrict__ weights,
                                                               const pulsar_block_q8_K *__restrict__ act, uint32_t nb,
                                                               uint32_t n_rows, uint32_t n_used, uint64_t row_bytes,
-                                                              uint32_t act_op) {
+                                                              uint32_t act_op, uint32_t shared_only) {
     using GT = GroupTile<Q, PAIR, NS>;
     __shared__ __align__(16) uint8_t buf0[GT::T::kBuf];
     __shared__ __align__(16) uint8_t buf1[GT::T::kBuf];
     __shared__ uint32_t pr_l[GT::T::kTok];
     extern __shared__ uint32_t lst[];
-    const ExpertGroups::Group grp = src.group(blockIdx.y);
+    const ExpertGroups::Group grp = shared_only ? src.shared_group(blockIdx.y) : src.group(blockIdx.y);
     const pulsar_expert_ptrs &p = grp.p;
     const bool nul = grp.is_null();  // block-uniform, as every exit below
     if (!nul && !(PAIR ? p.gate && p.up : p.down != nullptr)) return;
@@ -241,14 +242,16 @@ uint32_t tile_min_quarter_pairs(bool csr, bool pair, uint32_t quant, uint32_t nb
     F(PULSAR_QUANT_Q4_K) F(PULSAR_QUANT_Q5_K) F(PULSAR_QUANT_Q6_K) F(PULSAR_QUANT_Q2_K) F(PULSAR_QUANT_Q3_K)          \
     F(PULSAR_QUANT_IQ4_XS) F(PULSAR_QUANT_IQ2_XXS)
 
-// The grouped stages of an ExpertGroups source on the tile, n_group groups.
+// The grouped stages of an ExpertGroups source on the tile, n_group groups
+// (shared_only: the shared slots).
 int launch_tile_experts(bool pair, uint32_t quant, float *out, const ExpertGroups &src, const float *weights,
                         const pulsar_block_q8_K *act, uint32_t k_dim, uint32_t n_rows, uint32_t n_used,
-                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes) {
+                        uint32_t n_group, uint64_t row_bytes, uint32_t act_op, uint32_t lst_bytes, bool shared_only) {
 #define PK_LAUNCH(Q, P)                                                                                               \
     hipLaunchKernelGGL((tile_experts_kernel<Q, P, 4>),                                                                \
                        dim3((n_rows + GroupTile<Q, P, 4>::kRows - 1u) / GroupTile<Q, P, 4>::kRows, n_group), dim3(256), \
-                       lst_bytes, pk::stream(), out, src, weights, act, k_dim / 256u, n_rows, n_used, row_bytes, act_op)
+                       lst_bytes, pk::stream(), out, src, weights, act, k_dim / 256u, n_rows, n_used, row_bytes,      \
+                       act_op, (uint32_t)shared_only)
 #define PK_CASE(Q)                  \
     case Q:                         \
         if (pair)                   \
